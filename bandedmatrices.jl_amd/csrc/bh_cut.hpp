@@ -1,0 +1,118 @@
+// bh_cut.hpp -- a band recurrence cut into overlapping blocks that run at once.
+//
+// Band factorisations and solves are chains: step j needs what step j-1 left
+// in a window of the band's width, so one system keeps one workgroup (often
+// one wave) busy and the rest of the chip idle.  On matrices whose diagonal
+// dominates, that window forgets where the chain began: run from a wrong
+// state (none of the earlier steps), it reaches not only the same values to
+// rounding but the same bits after some 12 (FP64) or 8 (FP32) bandwidths --
+// an entry that differs in its last bit moves the entries it touches by far
+// less than half a bit of theirs.  So the n steps are cut into p blocks of L
+// steps; every block starts W steps early from the bare matrix, all blocks
+// run at once, and then the outcome is CHECKED: a block's factor columns (or
+// window) at its end must equal, bit for bit, what the next block computed
+// for the same steps before its own began.  The first block starts where the
+// chain starts, so equality at every seam makes every block's result the
+// sequential chain's, bit for bit.  If a seam differs nothing has been
+// written to the caller's arrays yet and the sequential kernel, launched
+// behind the blocks with the verdict as its condition, does the work.
+//
+// The check decides the result; the gate only decides whether trying is worth
+// its time (it samples columns for diagonal dominance: without it a matrix
+// that needs its pivots would pay for blocks that never agree).
+#pragma once
+#include "bh_common.hpp"
+
+namespace bh {
+
+// Device memory for one call, from a pool of the library's, ordered on the
+// stream: safe with any number of streams and threads.  The pool keeps at
+// most kCutKeep bytes between calls.  nullptr when there is none (or more
+// than kCutMax is asked for, or the stream is being captured): the caller
+// takes its sequential path.
+constexpr size_t kCutKeep = size_t(2) << 30;
+constexpr size_t kCutMax = size_t(8) << 30;
+void *cut_alloc(size_t bytes, hipStream_t st);
+void cut_free(void *p, hipStream_t st);
+// False when the environment says BANDEDHIP_CUT=off or a caller that may not
+// allocate has switched it off for this thread.
+bool cut_enabled();
+struct CutOff {  // no cutting on this thread while one of these lives
+    CutOff();
+    ~CutOff();
+};
+
+struct CutGeom {
+    int n, L, W, p;
+    __host__ __device__ int own(int i) const { return i * L; }
+    __host__ __device__ int start(int i) const { return i * L > W ? i * L - W : 0; }
+    __host__ __device__ int end(int i) const { return (i + 1) * L < n ? (i + 1) * L : n; }
+    __host__ __device__ int span() const { return L + W; }  // most steps of a block
+};
+
+// flags[0]: nonzero when the gate found the matrix not worth cutting;
+// flags[1]: nonzero when a seam differed or a block met a zero pivot.
+__device__ __forceinline__ bool cut_closed(const int *flags) { return __hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; }
+__device__ __forceinline__ bool cut_failed(const int *flags) {
+    return cut_closed(flags) || __hip_atomic_load(flags + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
+__device__ __forceinline__ bool cut_differ(double a, double b) {
+    return __builtin_bit_cast(unsigned long long, a) != __builtin_bit_cast(unsigned long long, b);
+}
+__device__ __forceinline__ bool cut_differ(float a, float b) {
+    return __builtin_bit_cast(unsigned, a) != __builtin_bit_cast(unsigned, b);
+}
+
+// One factorisation cut into blocks: block i factors columns start(i) ..
+// end(i)-1 and the rows they reach, in a copy of its own (ld = H = 2kl+ku+1),
+// as a system of its own.  g.p == 0: not cut (with flags: the sequential kernel
+// that runs only if the blocks failed).
+template <typename T>
+struct LuCut {
+    CutGeom g;
+    const int *flags;
+    T *ab;      // p copies of span() columns
+    i64 *ipiv;  // p runs of span() pivots, 1-based within the block
+    i64 *info;  // two words per block
+    int H, kl;
+    __device__ __forceinline__ T *block_ab(int i) const { return ab + (i64)i * g.span() * H; }
+    __device__ __forceinline__ int cols(int i) const { return g.end(i) - g.start(i); }
+    __device__ __forceinline__ int rows(int i) const {
+        const int e = g.end(i) + kl;
+        return (e < g.n ? e : g.n) - g.start(i);
+    }
+};
+
+// Gate: 256 columns spread over the matrix, 16 lanes to a column; closed when
+// more than a quarter of them have num/4 times the sum of |a| off the
+// diagonal above |a_jj|.  One workgroup, so it writes both flags itself.
+// The column's entries are rows r0 .. r0+h-1 of the band array, its diagonal
+// row d.
+constexpr int kCutSamples = 256;
+template <typename T>
+__global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, int r0, int h, int d, int num,
+                                                 int *flags) {
+    __shared__ int weak;
+    if (threadIdx.x == 0) weak = 0;
+    __syncthreads();
+    const int g = threadIdx.x >> 4, q = threadIdx.x & 15;
+    int mine = 0;
+#pragma unroll
+    for (int it = 0; it < kCutSamples / 64; ++it) {
+        const i64 c = ((i64)(64 * it + g) * n + n / 2) / kCutSamples;
+        const T *col = a + c * ld;
+        T s = T(0);
+        for (int r = q; r < h; r += 16) s += (r0 + r == d) ? T(0) : dabs(col[r0 + r]);
+        for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
+        mine += !(T(4) * dabs(col[d]) >= T(num) * s);
+    }
+    if (q == 0) atomicAdd(&weak, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        flags[0] = weak > kCutSamples / 4;
+        flags[1] = 0;
+    }
+}
+
+}  // namespace bh

@@ -14,6 +14,8 @@
 // entries are live) and the phases of a step are separated by workgroup
 // barriers.  Each phase is spread over the workgroup's lanes.
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
+#include "bh_lu_lane.hpp"
 
 #include <cstdlib>
 #include <cstring>
@@ -138,7 +140,8 @@ int blk_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i
 template <typename T>
 int small_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
 template <typename T>
-int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
+int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<T> *cut);
 
 // Kernel choice: BANDEDHIP_LU_KERNEL = "small" | "blk" | "reg" | "global" |
 // "mfma" forces one (where it applies).  By default, as LAPACK xGBTRF
@@ -161,6 +164,145 @@ static int lu_kernel_override() {
     return 0;
 }
 
+// ---------------------------------------------------------------- cut systems
+// (bh_cut.hpp).  The seams are checked on the multipliers and pivots alone:
+// at step t = c - (kl+ku) the rows still active hold nothing in columns >= c
+// yet (the rows read so far end before it), so two runs whose multipliers
+// and pivots agree over columns t .. c-1 do the same operations on the same
+// entries of every column from c on.
+
+// Copies of the blocks' columns, fill-in rows zeroed as LAPACK zeroes them
+// (slots outside the matrix keep what the caller has there).
+template <typename T>
+__global__ void __launch_bounds__(256) lu_cut_copy(LuCut<T> cut, const T *__restrict__ ab, i64 ld, int kv) {
+    if (cut_closed(cut.flags)) return;
+    const int blk = blockIdx.y, H = cut.H, s0 = cut.g.start(blk);
+    const int tot = cut.cols(blk) * H;
+    T *dst = cut.block_ab(blk);
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < tot; e += gridDim.x * 256) {
+        const int c = e / H, r = e - c * H;
+        const bool fill = r < cut.kl && s0 + c + r - kv >= 0;
+        dst[e] = fill ? T(0) : ab[(i64)(s0 + c) * ld + r];
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 2) cut.info[2 * blk + threadIdx.x] = 0;
+}
+
+// Block i against block i-1 over the `cmp` columns before its own begin.
+template <typename T>
+__global__ void __launch_bounds__(256) lu_cut_check(LuCut<T> cut, int kv, int cmp, int *flags) {
+    if (cut_closed(flags)) return;
+    const int blk = blockIdx.x, H = cut.H;
+    bool bad = threadIdx.x < 2 && cut.info[2 * blk + threadIdx.x] != 0;
+    if (cut.g.start(blk) > 0) {
+        const int c0 = cut.g.own(blk) - cmp, a0 = c0 - cut.g.start(blk - 1), b0 = c0 - cut.g.start(blk);
+        const T *a = cut.block_ab(blk - 1), *b = cut.block_ab(blk);
+        for (int e = threadIdx.x; e < cmp * cut.kl; e += 256) {
+            const int c = e / cut.kl, r = kv + 1 + e - c * cut.kl;
+            bad |= cut_differ(a[(i64)(a0 + c) * H + r], b[(i64)(b0 + c) * H + r]);
+        }
+        const i64 *pa = cut.ipiv + (i64)(blk - 1) * cut.g.span(), *pb = cut.ipiv + (i64)blk * cut.g.span();
+        for (int c = threadIdx.x; c < cmp; c += 256) bad |= pa[a0 + c] - a0 != pb[b0 + c] - b0;
+    }
+    if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(flags + 1, 1);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) lu_cut_commit(LuCut<T> cut, T *__restrict__ ab, i64 ld, i64 *__restrict__ ipiv) {
+    if (cut_failed(cut.flags)) return;
+    const int blk = blockIdx.y, H = cut.H, s0 = cut.g.start(blk), c0 = cut.g.own(blk), nc = cut.g.end(blk) - c0;
+    const T *src = cut.block_ab(blk) + (i64)(c0 - s0) * H;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < nc * H; e += gridDim.x * 256) {
+        const int c = e / H, r = e - c * H;
+        ab[(i64)(c0 + c) * ld + r] = src[e];
+    }
+    const i64 *pv = cut.ipiv + (i64)blk * cut.g.span() + (c0 - s0);
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256) ipiv[c0 + c] = pv[c] + s0;
+}
+
+static i64 up16(i64 x) { return (x + 15) & ~(i64)15; }
+
+// Blocks for n columns: W steps of lead-in, own steps so that `blocks` of
+// them fill the chip.  Measured over whole systems (n = 65536 and 262144,
+// bands from (1,1) to (128,128), N(0,1) + 2(kl+ku) I and U[0,1) + (kl+ku+1) I,
+// k = max(kl, ku)): every seam agrees from 8 k (FP32) and from 12 k (FP64) on
+// where kl = ku, earlier where they differ; 10 and 16 at k = 4.  A longer
+// lead-in costs little (FP64 (128,128): 3.15 ms at 12 k, 3.76 at 16 k, 58 ms
+// when it is too short), so some is added; `tries` times four.
+template <typename T>
+static CutGeom lu_cut_geom(i64 n, i64 kl, i64 ku, i64 blocks, int tries) {
+    const i64 k = imax(kl, ku);
+    i64 W = up16(imax(sizeof(T) == 8 ? 14 * k + 64 : 9 * k + 64, up16(kl + ku) + 16));
+    for (int t = 0; t < tries; ++t) W *= 4;
+    const i64 L = imax(64, up16(cdiv(n, blocks)));
+    CutGeom g{(int)n, (int)L, (int)W, (int)cdiv(n, L)};
+    // a block's L + W steps must be well under the chain's n
+    if (n >= (1ll << 29) || 3 * (L + W) > n) g.p = 0;
+    return g;
+}
+
+// Factor a square system by blocks.  Tried for sampled columns that exceed
+// 1.25 times the rest of their column: the measured families are at 2 and
+// more, and a matrix near 1 (the second difference) forgets too slowly for
+// its bits to agree, so it would only pay.  Measured, whole gbtrf call against the
+// sequential kernels: FP64 (8,8) n = 65536 0.40 ms against 31.3, (16,16)
+// n = 262144 1.7 against 125, (128,128) n = 65536 3.5 against 57.6 (FP32 2.0
+// against 37); what bounds it is the L + W steps of one block.  *ws: the blocks' memory with their
+// verdict in seq->flags, for the sequential kernel launched next (which does
+// nothing where the blocks succeeded) and to be freed after it; nullptr when
+// no blocks ran.
+template <typename T>
+static int gbtrf_cut(bool mfma, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, void **ws_out, LuCut<T> *seq) {
+    *ws_out = nullptr;
+    if (kl < 1 || !cut_enabled()) return BH_OK;
+    hipStream_t st = stream();
+    const int kv = (int)(kl + ku), H = (int)(2 * kl + ku + 1);
+    // one workgroup per CU for the MFMA kernel (its LDS), one wave per SIMD for the lane kernel
+    const i64 blocks = mfma ? 256 : 1024;
+    for (int tries = 0; tries < 2; ++tries) {
+        const CutGeom g = lu_cut_geom<T>(n, kl, ku, blocks, tries);
+        if (g.p == 0) return BH_OK;
+        const size_t ba = (((size_t)g.p * g.span() * H * sizeof(T)) + 255) & ~(size_t)255;
+        const size_t bp = (size_t)g.p * g.span() * sizeof(i64), bi = (size_t)g.p * 2 * sizeof(i64);
+        char *ws = (char *)cut_alloc(ba + bp + bi + 256, st);
+        if (!ws) return BH_OK;
+        int *flags = (int *)(ws + ba + bp + bi);
+        const LuCut<T> cut{g, flags, (T *)ws, (i64 *)(ws + ba), (i64 *)(ws + ba + bp), H, (int)kl};
+        hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n, (int)kl,
+                           (int)(kl + ku + 1), kv, 5, flags);
+        const unsigned gx = (unsigned)imin(64, cdiv((i64)g.span() * H, 1024));
+        hipLaunchKernelGGL(lu_cut_copy<T>, dim3(gx, g.p), dim3(256), 0, st, cut, (const T *)ab, ldab, kv);
+        int r = mfma ? mfma_gbtrf_launch<T>(n, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut)
+                     : lane_gbtrf_launch(n, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);
+        if (r != BH_OK) {
+            cut_free(ws, st);
+            return r == -1 ? BH_OK : r;  // -1: the kernel does not take this band
+        }
+        hipLaunchKernelGGL(lu_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, kv, (int)up16(kv), flags);
+        hipLaunchKernelGGL(lu_cut_commit<T>, dim3(gx, g.p), dim3(256), 0, st, cut, ab, ldab, ipiv);
+        hipError_t e = hipGetLastError();
+        // Long enough that four times the lead-in is still little of the
+        // chain: look at the verdict here (one wait) and try once more.
+        int fl[2] = {0, 0};
+        if (tries == 0 && n >= 32 * (i64)(g.L + 4 * g.W)) {
+            if (e == hipSuccess) e = hipMemcpyAsync(fl, flags, sizeof fl, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+        }
+        if (e != hipSuccess) {
+            cut_free(ws, st);
+            return hip_fail(e, "gbtrf (cut)", __FILE__, __LINE__);
+        }
+        if (fl[0] == 0 && fl[1] != 0) {
+            cut_free(ws, st);
+            continue;
+        }
+        *seq = LuCut<T>{};
+        seq->flags = flags;
+        *ws_out = ws;
+        return BH_OK;
+    }
+    return BH_OK;
+}
+
 template <typename T>
 static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *info_host) {
     BH_ARG(m >= 0, 1);
@@ -176,19 +318,41 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
         const int cs = ctrl_words(&dinfo);
         if (cs) return cs;
     }
-    BH_HIP(hipMemsetAsync(dinfo, 0, 2 * sizeof(i64), stream()));
     // register-resident kernel when the window fits one of its shapes,
     // otherwise the barrier-stepped kernel working in global memory
     const int ov = lu_kernel_override();
     int st = -1;
+    const bool mfma = ov == 5 || (ov == 0 && ((ku >= 65 && kl >= 32) || (kl >= 8 && ku >= 8 && imin(m, n) >= kLongLu)));
+    const bool lane = !mfma && ov == 0 && (kl <= 8 || kl == 16) && kl + ku <= 63 && !getenv("BANDEDHIP_SMALL_LU");
+    void *ws = nullptr;
+    LuCut<T> seq{};
+    if (m == n && (mfma || lane)) {
+        const int cs = gbtrf_cut<T>(mfma, n, kl, ku, ab, ldab, ipiv, &ws, &seq);
+        if (cs) return cs;
+    }
+    struct Free {
+        void *p;
+        ~Free() { cut_free(p, stream()); }
+    } free_ws{ws};
+    BH_HIP(hipMemsetAsync(dinfo, 0, 2 * sizeof(i64), stream()));
     // The MFMA-blocked factorisation (pivots equal xGBTF2's, factors to
     // rounding): where the reference itself runs blocked xGBTRF (ku >= 65,
     // kl >= 32), and for long systems with kl, ku >= 8, where the one-wave
     // chain of the narrow kernels is the longer path (n = 262144, (16,16):
     // 142 ms against 278 ms).  Shorter narrow systems keep the bit-exact
     // xGBTF2 kernels.
-    if (ov == 5 || (ov == 0 && ((ku >= 65 && kl >= 32) || (kl >= 8 && ku >= 8 && imin(m, n) >= kLongLu))))
-        st = mfma_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream());
+    if (mfma)
+        st = mfma_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), ws ? &seq : nullptr);
+    else if (ws)
+        st = lane_gbtrf_launch(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), &seq);
+    if (st == -1 && ws) {
+        // the blocks' kernel does not take the whole system (its 32-bit
+        // offsets): only their verdict tells whether another one has to run
+        int fl[2];
+        BH_HIP(hipMemcpyAsync(fl, seq.flags, sizeof fl, hipMemcpyDeviceToHost, stream()));
+        BH_HIP(hipStreamSynchronize(stream()));
+        if (fl[0] == 0 && fl[1] == 0) return BH_OK;
+    }
     // The one-wave lane kernel exists for kl <= 8 and kl = 16; above 16 the
     // blocked kernel beats the generic one-wave kernel (at n = 65536, (24,24):
     // 113.5 ms against 278.6 ms, identical factors), so it goes first there.

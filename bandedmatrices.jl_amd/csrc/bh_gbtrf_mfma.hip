@@ -48,6 +48,7 @@
 // sums in a different order than xGBTRF's DGEMM, so factors agree to
 // rounding, not bit for bit.
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 #include "bh_mfma.hpp"
 
 namespace bh {
@@ -74,6 +75,7 @@ struct QArgs {
     int m, n, kl, ku;
     i64 ldab;
     int R, RT, RP;  // window rows, 16-row tiles, padded rows (16*RT)
+    LuCut<T> cut;   // cut.g.p > 0: one workgroup per block of a cut system
 };
 
 template <typename T, int PR>
@@ -272,6 +274,18 @@ template <typename T, int PR>
 __global__ void __launch_bounds__(64 * QWAVES) gbtrf_mfma_kernel(QArgs<T> s) {
     using v4 = typename Mf<T>::v4;
     constexpr int QS = QStride<T>::value;
+    if (s.cut.g.p > 0) {  // this workgroup's block of a cut system
+        if (cut_closed(s.cut.flags)) return;
+        const int blk = blockIdx.x;
+        s.ab = s.cut.block_ab(blk);
+        s.ldab = s.cut.H;
+        s.m = s.cut.rows(blk);
+        s.n = s.cut.cols(blk);
+        s.ipiv = s.cut.ipiv + (i64)blk * s.cut.g.span();
+        s.info = s.cut.info + 2 * blk;
+    } else if (s.cut.flags && !cut_failed(s.cut.flags)) {
+        return;  // the blocks of a cut system have done it
+    }
     const int m = s.m, n = s.n, kl = s.kl, ku = s.ku, kv = kl + ku;
     const int R = s.R, RT = s.RT, RP = s.RP;
     const i64 ld = s.ldab;
@@ -755,7 +769,7 @@ int mfma_launch_one(const QArgs<T> &a, hipStream_t st) {
     auto kern = gbtrf_mfma_kernel<T, PR>;
     if (lds > 64 * 1024)
         BH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(1), dim3(64 * QWAVES), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.cut.g.p > 0 ? a.cut.g.p : 1), dim3(64 * QWAVES), lds, st, a);
     BH_LAUNCH_CHECK();
     return BH_OK;
 }
@@ -764,7 +778,8 @@ int mfma_launch_one(const QArgs<T> &a, hipStream_t st) {
 // step and those of column j+kv at step j (j < min(m,n)); zero them all up
 // front (rows whose row index is >= 0 only).
 template <typename T>
-__global__ void gbtrf_zero_fill(T *ab, i64 ld, int n, int mn, int kl, int ku) {
+__global__ void gbtrf_zero_fill(T *ab, i64 ld, int n, int mn, int kl, int ku, const int *flags) {
+    if (flags && !cut_failed(flags)) return;
     const int kv = kl + ku;
     const int c = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
     const int cend = qmin(n, mn + kv);
@@ -785,20 +800,25 @@ size_t mfma_lds_bytes(i64 kl, i64 elem) {
 // The blocked MFMA band LU, or -1 when the band does not fit it (kl + 16 rows
 // in at most four slots per lane and the LDS buffers, with the kernel's
 // static words (under 4 KiB), within 160 KiB).
+// With a cut it runs the blocks of a cut system in their own copies, whose
+// fill-in rows are already zero (ab, ipiv and dinfo are not read); with
+// cut->g.p == 0 it does nothing unless cut->flags say that the blocks failed.
 template <typename T>
-int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st) {
+int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<T> *cut) {
     const size_t lds = mfma_lds_bytes(kl, sizeof(T));
     if (lds == 0 || lds + 4096 > 160 * 1024 || m >= (1ll << 29) || n >= (1ll << 29) || kl + ku >= (1 << 20) ||
         (i64)QB * ldab * (i64)sizeof(T) >= (1ll << 31) || ldab * (i64)sizeof(T) >= (1ll << 24))
         return -1;
     const int R = (int)kl + QB, RT = (R + 15) / 16, RP = 16 * RT;
-    QArgs<T> a{ab, ipiv, dinfo, (int)m, (int)n, (int)kl, (int)ku, ldab, R, RT, RP};
+    QArgs<T> a{ab, ipiv, dinfo, (int)m, (int)n, (int)kl, (int)ku, ldab, R, RT, RP, LuCut<T>{}};
+    if (cut) a.cut = *cut;
     const int mn = (int)imin(m, n);
     const int cend = (int)imin(n, (i64)mn + kl + ku);
-    if (cend > ku + 1) {
+    if (a.cut.g.p == 0 && cend > ku + 1) {
         const int per = 4;  // columns per 256-thread block
         hipLaunchKernelGGL(gbtrf_zero_fill<T>, dim3((cend + per - 1) / per), dim3(64 * per), 0, st, ab, ldab, (int)n,
-                           mn, (int)kl, (int)ku);
+                           mn, (int)kl, (int)ku, a.cut.flags);
         BH_LAUNCH_CHECK();
     }
     const int PR = (R + 63) / 64;
@@ -816,7 +836,9 @@ int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
     }
 }
 
-template int mfma_gbtrf_launch<double>(i64, i64, i64, i64, double *, i64, i64 *, i64 *, hipStream_t);
-template int mfma_gbtrf_launch<float>(i64, i64, i64, i64, float *, i64, i64 *, i64 *, hipStream_t);
+template int mfma_gbtrf_launch<double>(i64, i64, i64, i64, double *, i64, i64 *, i64 *, hipStream_t,
+                                       const LuCut<double> *);
+template int mfma_gbtrf_launch<float>(i64, i64, i64, i64, float *, i64, i64 *, i64 *, hipStream_t,
+                                      const LuCut<float> *);
 
 }  // namespace bh

@@ -16,6 +16,7 @@
 // files see only the descriptor and the launchers.
 #pragma once
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 #include <type_traits>
 
@@ -29,9 +30,13 @@ struct BatchDesc {
 };
 
 // Single-system gbtrf through the rotating-register kernel (kl <= 8 or
-// kl = 16, kl + ku <= 63, band storage under 2 GiB), or -1.
-int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, double *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
-int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, float *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
+// kl = 16, kl + ku <= 63, band storage under 2 GiB), or -1.  With a cut it
+// runs the blocks of a cut system, one wave each; with cut->g.p == 0 it does
+// nothing unless cut->flags say that the blocks failed.
+int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, double *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<double> *cut);
+int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, float *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<float> *cut);
 // The persistent batched gbsv kernel over a schedule of nsys descriptors.
 int lane_batch_launch(unsigned blocks, unsigned threads, hipStream_t st, const BatchDesc *desc, int nsys, double *AB,
                       double *B, i64 *ipiv, i64 *info);
@@ -339,7 +344,20 @@ __device__ __forceinline__ int lane_gbsv_wave(int m, int n, int ku, T *__restric
 }
 
 template <typename T, int KL>
-__global__ void __launch_bounds__(64) gbtrf_lane_kernel(int m, int n, int ku, T *ab, i64 ld, i64 *ipiv, i64 *info) {
+__global__ void __launch_bounds__(64) gbtrf_lane_kernel(int m, int n, int ku, T *ab, i64 ld, i64 *ipiv, i64 *info,
+                                                        LuCut<T> cut) {
+    if (cut.g.p > 0) {  // this wave's block of a cut system
+        if (cut_closed(cut.flags)) return;
+        const int blk = blockIdx.x;
+        ab = cut.block_ab(blk);
+        ld = cut.H;
+        m = cut.rows(blk);
+        n = cut.cols(blk);
+        ipiv = cut.ipiv + (i64)blk * cut.g.span();
+        info = cut.info + 2 * blk;
+    } else if (cut.flags && !cut_failed(cut.flags)) {
+        return;  // the blocks of a cut system have done it
+    }
     const int r = lane_gbsv_wave<T, KL, false, 16>(m, n, ku, ab, ld, ipiv, nullptr);
     if (threadIdx.x == 0) *info = r;
 }
@@ -409,15 +427,19 @@ __global__ void __launch_bounds__(256) gbsv_batched_kernel(const BatchDesc *__re
 
 }  // namespace
 
-int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st) {
+int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<BH_LANE_T> *cut) {
     using T = BH_LANE_T;
-    if (kl + ku > 63 || m >= (1ll << 30) || n >= (1ll << 30) || ldab * n * (i64)sizeof(T) >= (1ll << 31)) return -1;
+    const i64 nb = cut && cut->g.p > 0 ? cut->g.span() : n;  // a block's copy holds span() columns
+    if (kl + ku > 63 || m >= (1ll << 30) || n >= (1ll << 30) || ldab * nb * (i64)sizeof(T) >= (1ll << 31)) return -1;
     const int mi = (int)m, ni = (int)n, ui = (int)ku;
+    const LuCut<T> c = cut ? *cut : LuCut<T>{};
+    const dim3 grid(c.g.p > 0 ? (unsigned)c.g.p : 1u);
     switch ((int)kl) {
 #define BH_LANE_CASE(KLv)                                                                                       \
     case KLv:                                                                                                   \
-        hipLaunchKernelGGL((gbtrf_lane_kernel<T, KLv>), dim3(1), dim3(64), 0, st, mi, ni, ui, ab, ldab, ipiv, \
-                           dinfo);                                                                              \
+        hipLaunchKernelGGL((gbtrf_lane_kernel<T, KLv>), grid, dim3(64), 0, st, mi, ni, ui, ab, ldab, ipiv,      \
+                           dinfo, c);                                                                           \
         break;
         BH_LANE_CASE(0) BH_LANE_CASE(1) BH_LANE_CASE(2) BH_LANE_CASE(3) BH_LANE_CASE(4)
         BH_LANE_CASE(5) BH_LANE_CASE(6) BH_LANE_CASE(7) BH_LANE_CASE(8) BH_LANE_CASE(16)

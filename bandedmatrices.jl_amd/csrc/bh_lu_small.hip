@@ -277,7 +277,7 @@ int small_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv,
     const int mi = (int)m, ni = (int)n, li = (int)kl, ui = (int)ku;
     const char *e = getenv("BANDEDHIP_SMALL_LU");
     if (!(e && strcmp(e, "class") == 0)) {
-        const int r = lane_gbtrf_launch(m, n, kl, ku, ab, ldab, ipiv, dinfo, st);
+        const int r = lane_gbtrf_launch(m, n, kl, ku, ab, ldab, ipiv, dinfo, st, nullptr);
         if (r != -1) return r;
     }
 #define BH_SMALL_CASE(C, RLv)                                                                                  \

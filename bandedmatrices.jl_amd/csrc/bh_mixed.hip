@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 namespace bh {
 
@@ -238,6 +239,7 @@ int bh_dsgbsv_noalloc(bh_int n, bh_int kl, bh_int ku, bh_int nrhs, const double 
         return BH_ERR_NODEVICE;
     }
     void *p = g_noalloc_ptr[dev];
+    const CutOff no_cut;  // the cut paths take device memory
     // the fallback overlays the refinement's workspace: by then it is dead
     return dsgbsv_impl(n, kl, ku, nrhs, A, lda, B, ldb, X, ldx, p, kNoAllocBytes, p, ipiv32, iters_host, info_host);
 }

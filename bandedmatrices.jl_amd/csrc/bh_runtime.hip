@@ -2,7 +2,13 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <stdlib.h>
+#include <string.h>
+
+#include <mutex>
+
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 namespace bh {
 
@@ -66,6 +72,66 @@ int scratch_buffer(size_t bytes, void **p) {
     }
     *p = g_scratch;
     return BH_OK;
+}
+
+// ---- memory of the cut paths (bh_cut.hpp): one stream-ordered pool per device
+constexpr int kCutDevices = 64;
+static hipMemPool_t g_cut_pool[kCutDevices] = {};
+static bool g_cut_none[kCutDevices] = {};
+static std::mutex g_cut_mutex;
+static thread_local int g_cut_off = 0;
+
+CutOff::CutOff() { ++g_cut_off; }
+CutOff::~CutOff() { --g_cut_off; }
+
+bool cut_enabled() {
+    if (g_cut_off > 0) return false;
+    const char *e = getenv("BANDEDHIP_CUT");
+    return !(e && !strcmp(e, "off"));
+}
+
+static hipMemPool_t cut_pool(int dev) {
+    std::lock_guard<std::mutex> lock(g_cut_mutex);
+    if (g_cut_pool[dev] || g_cut_none[dev]) return g_cut_pool[dev];
+    hipMemPoolProps props;
+    memset(&props, 0, sizeof props);
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    hipMemPool_t pool = nullptr;
+    hipError_t e = hipMemPoolCreate(&pool, &props);
+    if (e == hipSuccess) {
+        uint64_t keep = kCutKeep;
+        e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        g_cut_none[dev] = true;
+        return nullptr;
+    }
+    return g_cut_pool[dev] = pool;
+}
+
+void *cut_alloc(size_t bytes, hipStream_t st) {
+    if (bytes > kCutMax) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    int dev = -1;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= kCutDevices) return nullptr;
+    hipMemPool_t pool = cut_pool(dev);
+    void *p = nullptr;
+    if (!pool || hipMallocFromPoolAsync(&p, bytes, pool, st) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+void cut_free(void *p, hipStream_t st) {
+    if (p && hipFreeAsync(p, st) != hipSuccess) (void)hipGetLastError();
 }
 
 }  // namespace bh

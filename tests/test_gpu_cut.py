@@ -1,0 +1,79 @@
+"""GPU: systems cut into blocks that run at once (csrc/bh_cut.hpp) against the
+same entry points with cutting switched off.  Whether a system is cut and its
+seams agree, or the sequential kernels run, the outputs are the same bits: the
+lead-in's rounding is checked, not trusted.  Inputs that must fall back (weak
+diagonals, a zero column, a NaN, interchanges) are mixed with dominant ones,
+at sizes around the edges of the blocks."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from _util import band
+
+pytestmark = pytest.mark.gpu
+
+FP = {np.float64: "d", np.float32: "s"}
+
+
+def _both(monkeypatch, f):
+    """f() with cutting allowed and with it off."""
+    monkeypatch.delenv("BANDEDHIP_CUT", raising=False)
+    on = f()
+    monkeypatch.setenv("BANDEDHIP_CUT", "off")
+    off = f()
+    return on, off
+
+
+def _same(on, off):
+    for a, b in zip(on, off):
+        if isinstance(a, np.ndarray):
+            assert a.shape == b.shape and a.tobytes() == b.tobytes(), np.argwhere(a != b)[:5]
+        else:
+            assert a == b
+
+
+def _system(rng, n, kl, ku, dtype, kind):
+    A = band(rng, kl, ku, n, np.float64, dist="n")
+    A[ku, :] += 2 * (kl + ku) + 2
+    if kind == "weak":  # a stretch whose diagonal does not dominate: interchanges, and slow or no agreement
+        A[ku, n // 3 : n // 3 + 200] -= 2 * (kl + ku) + 2
+    elif kind == "zero":
+        A[:, n // 2] = 0
+    elif kind == "nan":
+        A[ku, n // 2] = np.nan
+    elif kind == "random":
+        A = band(rng, kl, ku, n, np.float64, dist="u")
+    return np.asfortranarray(A.astype(dtype))
+
+
+LU = [  # n, kl, ku: lane kernel, its edges; the MFMA kernel for long and for wide bands
+    (1000, 1, 1), (1003, 2, 5), (4096, 4, 4), (10000, 4, 3), (10001, 8, 8), (5000, 16, 3), (16383, 8, 8),
+    (16384, 8, 8), (16400, 16, 16), (262144, 9, 9), (30001, 9, 20), (9000, 64, 70), (12345, 100, 128), (3000, 33, 65),
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["dominant", "weak", "zero", "nan", "random"])
+@pytest.mark.parametrize("n,kl,ku", LU)
+def test_lu(bh, monkeypatch, dtype, kind, n, kl, ku):
+    if kind != "dominant" and n > 12000:
+        pytest.skip("the fallbacks are the same code at every length")
+    print(f"lu {dtype.__name__} {kind} n={n} ({kl},{ku})", flush=True)
+    A = _system(np.random.default_rng(n + kl), n, kl, ku, dtype, kind)
+    ld = 2 * kl + ku + 2  # a leading dimension one larger than the band
+    ab = np.full((ld, n), 7, dtype, order="F")
+    ab[kl : 2 * kl + ku + 1] = A
+
+    def run():
+        d = bh.DeviceArray.from_numpy(ab)
+        ipiv, info = bh.DeviceArray((n,), np.int64), C.c_int64(-7)
+        bh._lib.call(f"bh_{FP[dtype]}gbtrf", n, n, kl, ku, d.ptr, ld, ipiv.ptr, C.byref(info))
+        f, p = d.numpy(), ipiv.numpy()
+        # pivots and columns past a zero pivot are defined, those past a NaN compare by bits too
+        return f, p, info.value
+
+    on, off = _both(monkeypatch, run)
+    if kind == "dominant":
+        assert off[2] == 0
+    _same(on, off)
