@@ -77,3 +77,43 @@ def test_lu(bh, monkeypatch, dtype, kind, n, kl, ku):
     if kind == "dominant":
         assert off[2] == 0
     _same(on, off)
+
+
+def _triangle(rng, n, k, up, dtype, kind):
+    A = rng.uniform(-1, 1, (k + 1, n)) * (0.5 / max(k, 1))
+    d = k if up else 0
+    A[d] = 1 + rng.random(n)
+    if kind == "weak":
+        A[d, n // 3 : n // 3 + 300] = 0.01
+    elif kind == "zero":
+        A[d, n // 2] = 0
+    elif kind == "nan":
+        A[(d + 1) % (k + 1), n // 2] = np.nan
+    return np.asfortranarray(A.astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo,trans", [("U", "N"), ("L", "N"), ("U", "T"), ("L", "T")])
+@pytest.mark.parametrize("kind", ["dominant", "weak", "zero", "nan"])
+@pytest.mark.parametrize("n,k,nrhs,incx,diag", [
+    (3000, 1, 1, 1, "N"), (4097, 3, 3, 1, "N"), (20000, 8, 1, 2, "U"), (20031, 16, 2, 1, "N"), (30000, 64, 1, 1, "N"),
+    (40001, 100, 2, 1, "U"), (66000, 200, 1, 1, "N"), (5000, 0, 1, 1, "N"),
+])
+def test_triangular(bh, monkeypatch, dtype, uplo, trans, kind, n, k, nrhs, incx, diag):
+    if kind == "nan" and k == 0:
+        pytest.skip("a diagonal matrix has no chain")
+    print(f"tbsv {dtype.__name__} {uplo}{trans}{diag} {kind} n={n} k={k} nrhs={nrhs} incx={incx}", flush=True)
+    rng = np.random.default_rng(n + k)
+    A = bh.DeviceArray.from_numpy(_triangle(rng, n, k, uplo == "U", dtype, kind))
+    b = rng.standard_normal(n * incx if nrhs == 1 else (n + 3, nrhs)).astype(dtype)
+    p, u, t, d = FP[dtype], uplo.encode(), trans.encode(), diag.encode()
+
+    def run():
+        x = bh.DeviceArray.from_numpy(b)
+        if nrhs == 1:
+            bh._lib.call(f"bh_{p}tbsv", u, t, d, n, k, A.ptr, A.ld, x.ptr, incx)
+        else:
+            bh._lib.call(f"bh_{p}tbsv_multi", u, t, d, n, k, A.ptr, A.ld, nrhs, x.ptr, n + 3)
+        return (x.numpy(),)
+
+    _same(*_both(monkeypatch, run))
