@@ -25,7 +25,16 @@
 // only.  Incoming columns arrive in chunks of B: a chunk is loaded into
 // registers while the previous one is consumed and stored to LDS when it is
 // done, so no step waits on HBM.
+//
+// Where the diagonal dominates, the columns are cut into blocks that start a
+// lead-in early, each in a workgroup of its own (bh_cut.hpp).  The kernel
+// reads every column once and writes it once, so a block reads the caller's
+// array and writes to a copy.  Its seams are checked on the kd factor columns
+// before each block's own: at step c - kd no earlier column has touched a row
+// and column >= c, so two runs whose rows of U over steps c-kd .. c-1 agree
+// up to column c-1 leave the same entries from there on.
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 #include "bh_tbsv.hpp"
 
 namespace bh {
@@ -40,8 +49,37 @@ __device__ __forceinline__ float dsqrt<float>(float x) { return __builtin_sqrtf(
 
 constexpr int kPbRegs = 24;  // staged values per thread: chunk columns x (kd+1) <= kPbRegs x threads
 
+// One factorisation by blocks; g.p == 0: the whole of it (with flags: only if
+// the blocks failed).
+template <typename T>
+struct PbCut {
+    CutGeom g;
+    const int *flags;
+    T *out;     // p copies of span() + kd columns of kd+1 rows
+    i64 *info;  // one word per block
+    // columns a block runs: a lower factor's last own columns reach kd rows
+    // further, into the next block
+    __device__ __forceinline__ int cols(int i, int kd, bool up) const {
+        const int e = g.end(i) + (up ? 0 : kd);
+        return (e < g.n ? e : g.n) - g.start(i);
+    }
+    __device__ __forceinline__ T *block(int i, int kd) const { return out + (i64)i * (g.span() + kd) * (kd + 1); }
+};
+
 template <typename T, bool UP, bool LDL>
-__global__ void __launch_bounds__(256) pbtrf_lds_kernel(int n, int kd, T *__restrict__ ab, i64 ldab, i64 *__restrict__ info_out, int B) {
+__global__ void __launch_bounds__(256) pbtrf_lds_kernel(int n, int kd, const T *ab, i64 ldab, T *out, i64 ldo,
+                                                        i64 *__restrict__ info_out, int B, PbCut<T> cut) {
+    if (cut.g.p > 0) {
+        if (cut_closed(cut.flags)) return;
+        const int blk = blockIdx.x;
+        ab += (i64)cut.g.start(blk) * ldab;
+        n = cut.cols(blk, kd, UP);
+        out = cut.block(blk, kd);
+        ldo = kd + 1;
+        info_out = cut.info + blk;
+    } else if (cut.flags && !cut_failed(cut.flags)) {
+        return;
+    }
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int H = kd + 1;
     // slot stride: even, so that entries one row apart in neighbouring slots
@@ -140,7 +178,7 @@ __global__ void __launch_bounds__(256) pbtrf_lds_kernel(int n, int kd, T *__rest
             // column j is final: write it out; its slot takes column j+kd+1 from S
             T *sj = slot(j);
             if (tid < H) {
-                ab[(i64)j * ldab + tid] = sj[tid];
+                out[(i64)j * ldo + tid] = sj[tid];
                 if (j + H < n) sj[tid] = S[(j - j0) * H + tid];
             }
             // kd == 0: no update ran, and column j+1 has just entered slot(j)
@@ -158,9 +196,52 @@ __global__ void __launch_bounds__(256) pbtrf_lds_kernel(int n, int kd, T *__rest
     // stopped early: the columns still in the window go back as they stand
     if (done < n) {
         for (int c = done; c < min(n, done + H); ++c)
-            for (int r = tid; r < H; r += nt) ab[(i64)c * ldab + r] = slot(c)[r];
+            for (int r = tid; r < H; r += nt) out[(i64)c * ldo + r] = slot(c)[r];
     }
     if (tid == 0) *info_out = sInfo;
+}
+
+// block i against block i-1 over the kd columns before its own; a row past
+// the last of them is block i's alone
+template <typename T>
+__global__ void __launch_bounds__(256) pb_cut_check(PbCut<T> cut, int kd, int up, int *flags) {
+    if (cut_closed(flags)) return;
+    const int blk = blockIdx.x, H = kd + 1;
+    bool bad = threadIdx.x == 0 && cut.info[blk] != 0;
+    if (cut.g.start(blk) > 0) {
+        const int c0 = cut.g.own(blk) - kd;
+        const T *a = cut.block(blk - 1, kd) + (i64)(c0 - cut.g.start(blk - 1)) * H;
+        const T *b = cut.block(blk, kd) + (i64)(c0 - cut.g.start(blk)) * H;
+        for (int e = threadIdx.x; e < kd * H; e += 256)
+            if (up || e / H + e % H < kd) bad |= cut_differ(a[e], b[e]);
+    }
+    if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(flags + 1, 1);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) pb_cut_commit(PbCut<T> cut, int kd, T *__restrict__ ab, i64 ldab) {
+    if (cut_failed(cut.flags)) return;
+    const int blk = blockIdx.y, H = kd + 1, c0 = cut.g.own(blk), nc = cut.g.end(blk) - c0;
+    const T *src = cut.block(blk, kd) + (i64)(c0 - cut.g.start(blk)) * H;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < nc * H; e += gridDim.x * 256) {
+        const int c = e / H, r = e - c * H;
+        ab[(i64)(c0 + c) * ldab + r] = src[e];
+    }
+}
+
+// Blocks of a Cholesky or LDL' factorisation: lead-in measured at diagonals
+// kd+1 .. kd+2 under entries U(-1,1) (kd = 2 .. 64): the bits agree after
+// 8-12 kd columns in FP64 and 4-6 kd in FP32; four blocks to a CU (small
+// windows: their barriers overlap), not under half the lead-in each.  Factor
+// and solve at n = 65536, kd = 8, FP64: 73.7 -> 0.71 ms; the chain of one
+// block (L + W steps of 1.1 us) bounds it.
+template <typename T>
+CutGeom pb_cut_geom(i64 n, i64 kd) {
+    const i64 W = (sizeof(T) == 8 ? 14 : 8) * kd + 32;
+    const i64 L = imax(cdiv(n, 1024), W / 2);
+    CutGeom g{(int)n, (int)L, (int)W, (int)cdiv(n, L)};
+    if (kd < 1 || 3 * (L + W) > n) g.p = 0;
+    return g;
 }
 
 template <typename T, bool LDL>
@@ -195,10 +276,37 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
     }
     auto kern = up ? pbtrf_lds_kernel<T, true, LDL> : pbtrf_lds_kernel<T, false, LDL>;
     hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // By blocks where |a_jj| is at least 1.75 times the sum of its stored
+    // row or column (half of the off-diagonal entries: plain dominance is 2
+    // on average); behind them the whole chain, which does nothing where the
+    // blocks agreed.
+    PbCut<T> cut{};
+    char *ws = nullptr;
+    const CutGeom g = pb_cut_geom<T>(n, kd);
+    if (e == hipSuccess && g.p > 0 && cut_enabled()) {
+        const size_t bo = ((size_t)g.p * (g.span() + kd) * H * sizeof(T) + 255) & ~(size_t)255;
+        const size_t bi = (size_t)g.p * sizeof(i64);
+        ws = (char *)cut_alloc(bo + bi + 256, st);
+        if (ws) {
+            int *flags = (int *)(ws + bo + bi);
+            cut = PbCut<T>{g, flags, (T *)ws, (i64 *)(ws + bo)};
+            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n, 0, (int)H,
+                               up ? (int)kd : 0, 0, 7, flags, 0);
+            hipLaunchKernelGGL(kern, dim3(g.p), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, (T *)nullptr,
+                               (i64)0, (i64 *)nullptr, (int)B, cut);
+            hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, (int)kd, (int)up, flags);
+            hipLaunchKernelGGL(pb_cut_commit<T>, dim3((unsigned)imin(16, cdiv(g.L * H, 256)), g.p), dim3(256), 0, st,
+                               cut, (int)kd, ab, ldab);
+            e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
+            cut.g.p = 0;
+        }
+    }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(kern, dim3(1), dim3(nt), lds, st, (int)n, (int)kd, ab, ldab, dinfo, (int)B);
+        hipLaunchKernelGGL(kern, dim3(1), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, ab, ldab, dinfo,
+                           (int)B, cut);
         e = hipGetLastError();
     }
+    cut_free(ws, st);
     if (e == hipSuccess) e = hipMemcpyAsync(info_host, dinfo, sizeof(i64), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(e, "pbtrf", __FILE__, __LINE__);

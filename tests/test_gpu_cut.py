@@ -117,3 +117,36 @@ def test_triangular(bh, monkeypatch, dtype, uplo, trans, kind, n, k, nrhs, incx,
         return (x.numpy(),)
 
     _same(*_both(monkeypatch, run))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("ldl", [False, True])
+@pytest.mark.parametrize("kind", ["dominant", "weak", "zero", "nan"])
+@pytest.mark.parametrize("n,kd", [(500, 1), (1003, 2), (4096, 8), (9001, 17), (12000, 64), (30000, 128)])
+def test_cholesky(bh, monkeypatch, dtype, uplo, ldl, kind, n, kd):
+    if kd > 120 and (dtype == np.float64 or kind != "dominant"):
+        pytest.skip("the LDS window holds it in single precision; one long chain is enough")
+    print(f"cholesky {dtype.__name__} {uplo} ldl={ldl} {kind} n={n} kd={kd}", flush=True)
+    rng = np.random.default_rng(n + kd)
+    A = rng.uniform(-1, 1, (kd + 1, n))
+    d = kd if uplo == "U" else 0
+    A[d] = kd + 2 + rng.random(n)
+    if kind == "weak":  # not positive definite there: info > 0, or no agreement
+        A[d, n // 3 : n // 3 + 40] = 0.3
+    elif kind == "zero":
+        A[d, n // 2] = 0
+    elif kind == "nan":
+        A[d, n // 2] = np.nan
+    ab = np.full((kd + 3, n), 5, dtype, order="F")
+    ab[: kd + 1] = A
+
+    def run():
+        x, info = bh.DeviceArray.from_numpy(ab), C.c_int64(-7)
+        if ldl:
+            bh._lib.call(f"bh_{FP[dtype]}sbldlt", uplo.encode(), n, kd, x.ptr, kd + 3)
+            return x.numpy(), 0
+        bh._lib.call(f"bh_{FP[dtype]}pbtrf", uplo.encode(), n, kd, x.ptr, kd + 3, C.byref(info))
+        return x.numpy(), info.value
+
+    _same(*_both(monkeypatch, run))
