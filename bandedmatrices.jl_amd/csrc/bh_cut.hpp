@@ -25,9 +25,10 @@
 
 namespace bh {
 
-// Device memory for one call, from a pool of the library's, ordered on the
-// stream: safe with any number of streams and threads.  The pool keeps at
-// most kCutKeep bytes between calls.  nullptr when there is none (or more
+// Device memory for one call on this thread's buffer for the stream, used in the
+// stream's order until cut_free: safe with any number of streams and threads.
+// A thread keeps at most four buffers of kCutKeep bytes and frees them when it
+// ends; larger ones go back at once.  nullptr when there is none (or more
 // than kCutMax is asked for, or the stream is being captured): the caller
 // takes its sequential path.
 constexpr size_t kCutKeep = size_t(2) << 30;
@@ -87,30 +88,40 @@ struct LuCut {
 // Gate: 256 columns spread over the matrix, 16 lanes to a column; closed when
 // more than a quarter of them have num/4 times the sum of |a| off the
 // diagonal above |a_jj|.  One workgroup, so it writes both flags itself.
-// The column's entries are rows r0 .. r0+h-1 of the band array, its diagonal
-// row d (with `unit` it counts as 1).  `more`: a second gate of the same call.
+// A set of entries of a column: rows r0 .. r0+h-1 of the band array, the
+// diagonal in row d (with `unit` it counts as 1); h = 0: no second set.
+struct CutSet {
+    int r0, h, d, unit;
+};
 constexpr int kCutSamples = 256;
 template <typename T>
-__global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, int r0, int h, int d, int unit,
-                                                 int num, int *flags, int more) {
-    __shared__ int weak;
-    if (threadIdx.x == 0) weak = 0;
+__global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, CutSet s1, CutSet s2, int num,
+                                                 int *flags) {
+    __shared__ int weak[2];
+    if (threadIdx.x < 2) weak[threadIdx.x] = 0;
     __syncthreads();
     const int g = threadIdx.x >> 4, q = threadIdx.x & 15;
-    int mine = 0;
+    int m1 = 0, m2 = 0;
+    auto strong = [&](const T *col, const CutSet &s) {
+        T t = T(0);
+        for (int r = q; r < s.h; r += 16) t += (s.r0 + r == s.d) ? T(0) : dabs(col[s.r0 + r]);
+        for (int off = 8; off > 0; off >>= 1) t += __shfl_xor(t, off, 16);
+        return T(4) * (s.unit ? T(1) : dabs(col[s.d])) >= T(num) * t;
+    };
 #pragma unroll
     for (int it = 0; it < kCutSamples / 64; ++it) {
         const i64 c = ((i64)(64 * it + g) * n + n / 2) / kCutSamples;
         const T *col = a + c * ld;
-        T s = T(0);
-        for (int r = q; r < h; r += 16) s += (r0 + r == d) ? T(0) : dabs(col[r0 + r]);
-        for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
-        mine += !(T(4) * (unit ? T(1) : dabs(col[d])) >= T(num) * s);
+        m1 += !strong(col, s1);
+        if (s2.h) m2 += !strong(col, s2);
     }
-    if (q == 0) atomicAdd(&weak, mine);
+    if (q == 0) {
+        atomicAdd(&weak[0], m1);
+        atomicAdd(&weak[1], m2);
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        flags[0] = (more ? flags[0] : 0) | (weak > kCutSamples / 4);
+        flags[0] = weak[0] > kCutSamples / 4 || weak[1] > kCutSamples / 4;
         flags[1] = 0;
     }
 }
@@ -128,6 +139,13 @@ struct SweepCut {
     __device__ __forceinline__ T *at(int blk, int which, int cnt) const {
         return snap + (((i64)blk * gridDim.x + blockIdx.x) * 2 + which) * cnt;
     }
+};
+
+// The memory of a solve by blocks alone (nullptr: none ran) and its verdict,
+// freed by whoever asked for it after reading the flags.
+struct RingCutWs {
+    void *ws = nullptr;
+    const int *flags = nullptr;
 };
 
 // cnt entries per window; grid (p - 1, nrhs)

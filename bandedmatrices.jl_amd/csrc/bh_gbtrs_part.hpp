@@ -26,8 +26,16 @@
 #pragma once
 
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 namespace bh {
+
+template <typename T>
+int ring_gbtrs_launch(int how, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
+                      hipStream_t st, RingCutWs *cw);
+template <typename T>
+int ring_gbtrs_t_launch(int how, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
+                        hipStream_t st, RingCutWs *cw);
 
 namespace part {
 
@@ -53,6 +61,7 @@ struct PartArgs {
     unsigned *growth;  // largest |entry| of the A_i (FP32 bits, NaN above all), per sweep
     i64 ld, ldb, ldy;
     int n, kl, kv, nrhs, M, p;
+    const int *skip;  // verdict of a solve by blocks launched before: nothing runs where it stands
 };
 
 template <int K>
@@ -83,6 +92,7 @@ __device__ __forceinline__ int prow(int js, int je, int s) {
 // blockIdx.y = g the right-hand sides 16g .. from the true state.
 template <typename T, int KW, int OP, bool FINAL>
 __global__ void __launch_bounds__(64) part_run(PartArgs<T> a) {
+    if (a.skip && !cut_failed(a.skip)) return;
     constexpr int G = (64 + KW - 1) / KW;
     constexpr int CHS = G * KW;  // steps per staged chunk (whole groups of KW)
     const int lane = threadIdx.x;
@@ -264,6 +274,7 @@ struct PChain {
 
 template <typename T, int KW, int OP>
 __global__ void __launch_bounds__(256) part_chain(PartArgs<T> a, int RB) {
+    if (a.skip && !cut_failed(a.skip)) return;
     using C = PChain<T, KW>;
     constexpr int MPER = C::MPER, PD = C::PD, AS = C::AS;
     const int tid = threadIdx.x;
@@ -515,6 +526,22 @@ int part_solve(char trans, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 lda
         a.cvec = a.dvec + (size_t)p.p * nrhs * p.KW;
     };
     const bool tr = trans != 'N';
+    // The sequential sweeps by blocks first (bh_gbtrs_ring.hpp): where the
+    // factors are dominant they take an eighth of the transfer matrices' time and have
+    // the exact solve's bits.  What follows is launched behind them, does
+    // nothing where they agreed, and shares its wait with their verdict.
+    RingCutWs cw;
+    {
+        const int r = tr ? ring_gbtrs_t_launch<T>(2, n, kl, ku, nrhs, ab, ldab, ipiv, B, ldb, st, &cw)
+                         : ring_gbtrs_launch<T>(2, n, kl, ku, nrhs, ab, ldab, ipiv, B, ldb, st, &cw);
+        if (r != BH_OK && r != -1) return r;  // -1: a band or length it does not take
+    }
+    struct Free {
+        void *p;
+        hipStream_t st;
+        ~Free() { cut_free(p, st); }
+    } free_cw{cw.ws, st};
+    a.skip = cw.flags;
     a.growth = reinterpret_cast<unsigned *>(Y + (size_t)n * nrhs);
     hipLaunchKernelGGL(part_clear, dim3(1), dim3(64), 0, st, a.growth);
     BH_LAUNCH_CHECK();
@@ -555,7 +582,13 @@ int part_solve(char trans, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 lda
     if (stt) return stt;
     unsigned gh[2];
     BH_HIP(hipMemcpyAsync(gh, a.growth - 1, sizeof gh, hipMemcpyDeviceToHost, st));
+    int fl[2] = {1, 1};
+    if (cw.ws) BH_HIP(hipMemcpyAsync(fl, cw.flags, sizeof fl, hipMemcpyDeviceToHost, st));
     BH_HIP(hipStreamSynchronize(st));
+    if (fl[0] == 0 && fl[1] == 0) return BH_OK;  // B holds the blocks' solution
+    cut_free(cw.ws, st);
+    free_cw.p = nullptr;
+    a.skip = nullptr;
     const float g0 = __builtin_bit_cast(float, gh[0]), g1 = __builtin_bit_cast(float, gh[1]);
     if (!(g0 <= kPartGrowthMax<T>) || !(g1 <= kPartGrowthMax<T>)) {
         // the blocks amplify too much for the partitioned result: the sequential solve

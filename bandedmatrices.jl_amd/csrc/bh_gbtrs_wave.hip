@@ -16,6 +16,7 @@
 // 'T' backward: b_j -= sum_t l_{j+t,j} b_{j+t}; swap b_j <-> b_p
 //   -- dot products are wave reductions (summation order differs from BLAS).
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 #include <cstdlib>
 #include <cstring>
@@ -289,11 +290,11 @@ gbtrs_t_wave(i64 n, i64 kl, i64 ku, const T *__restrict__ ab, i64 ld, const i64 
 }
 
 template <typename T>
-int ring_gbtrs_launch(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
-                      hipStream_t st);
+int ring_gbtrs_launch(int how, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
+                      hipStream_t st, RingCutWs *cw);
 template <typename T>
-int ring_gbtrs_t_launch(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
-                        hipStream_t st);
+int ring_gbtrs_t_launch(int how, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B, i64 ldb,
+                        hipStream_t st, RingCutWs *cw);
 
 template <typename T>
 int wave_gbtrs_launch(bool trans_n, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B,
@@ -302,8 +303,8 @@ int wave_gbtrs_launch(bool trans_n, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab
     {
         const char *e = getenv("BANDEDHIP_TRS_KERNEL");
         if (!(e && !strcmp(e, "shift"))) {
-            const int r = trans_n ? ring_gbtrs_launch<T>(n, kl, ku, nrhs, ab, ld, ipiv, B, ldb, st)
-                                  : ring_gbtrs_t_launch<T>(n, kl, ku, nrhs, ab, ld, ipiv, B, ldb, st);
+            const int r = trans_n ? ring_gbtrs_launch<T>(1, n, kl, ku, nrhs, ab, ld, ipiv, B, ldb, st, nullptr)
+                                  : ring_gbtrs_t_launch<T>(1, n, kl, ku, nrhs, ab, ld, ipiv, B, ldb, st, nullptr);
             if (r != -1) return r;
         }
     }

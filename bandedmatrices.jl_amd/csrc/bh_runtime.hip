@@ -5,8 +5,6 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <mutex>
-
 #include "bh_common.hpp"
 #include "bh_cut.hpp"
 
@@ -74,42 +72,40 @@ int scratch_buffer(size_t bytes, void **p) {
     return BH_OK;
 }
 
-// ---- memory of the cut paths (bh_cut.hpp): one stream-ordered pool per device
-constexpr int kCutDevices = 64;
-static hipMemPool_t g_cut_pool[kCutDevices] = {};
-static bool g_cut_none[kCutDevices] = {};
-static std::mutex g_cut_mutex;
-static thread_local int g_cut_off = 0;
+// ---- memory of the cut paths (bh_cut.hpp).  Each thread keeps up to four
+// buffers of at most kCutKeep bytes, one to a stream, and frees them when it ends;
+// a fifth stream takes over the buffer unused for longest, behind its last
+// use.  (A stream-ordered pool of HIP's, tried first, cost 60-140 us a call
+// with a synchronisation between calls; this costs under 5.)
+struct CutBuf {
+    int dev = -1;
+    hipStream_t st = nullptr;
+    void *p = nullptr;
+    size_t bytes = 0;
+    hipEvent_t done = nullptr;  // behind the last call that used it
+    bool busy = false;
+    unsigned long long used = 0;
+};
+struct CutBufs {
+    CutBuf b[4];
+    unsigned long long clock = 0;
+    int off = 0;
+    ~CutBufs() {
+        for (CutBuf &c : b) {
+            if (c.p) (void)hipFree(c.p);
+            if (c.done) (void)hipEventDestroy(c.done);
+        }
+    }
+};
+static thread_local CutBufs g_cut;
 
-CutOff::CutOff() { ++g_cut_off; }
-CutOff::~CutOff() { --g_cut_off; }
+CutOff::CutOff() { ++g_cut.off; }
+CutOff::~CutOff() { --g_cut.off; }
 
 bool cut_enabled() {
-    if (g_cut_off > 0) return false;
+    if (g_cut.off > 0) return false;
     const char *e = getenv("BANDEDHIP_CUT");
     return !(e && !strcmp(e, "off"));
-}
-
-static hipMemPool_t cut_pool(int dev) {
-    std::lock_guard<std::mutex> lock(g_cut_mutex);
-    if (g_cut_pool[dev] || g_cut_none[dev]) return g_cut_pool[dev];
-    hipMemPoolProps props;
-    memset(&props, 0, sizeof props);
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = dev;
-    hipMemPool_t pool = nullptr;
-    hipError_t e = hipMemPoolCreate(&pool, &props);
-    if (e == hipSuccess) {
-        uint64_t keep = kCutKeep;
-        e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        g_cut_none[dev] = true;
-        return nullptr;
-    }
-    return g_cut_pool[dev] = pool;
 }
 
 void *cut_alloc(size_t bytes, hipStream_t st) {
@@ -120,18 +116,60 @@ void *cut_alloc(size_t bytes, hipStream_t st) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= kCutDevices) return nullptr;
-    hipMemPool_t pool = cut_pool(dev);
-    void *p = nullptr;
-    if (!pool || hipMallocFromPoolAsync(&p, bytes, pool, st) != hipSuccess) {
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    CutBuf *c = nullptr;
+    for (CutBuf &x : g_cut.b) {
+        if (x.busy) continue;
+        if (x.p && x.dev == dev && x.st == st) {
+            c = &x;
+            break;
+        }
+        if (!c || x.used < c->used) c = &x;
+    }
+    if (!c) return nullptr;
+    bool ok = true;
+    if (c->p && (c->dev != dev || c->bytes < bytes)) {
+        ok = hipEventSynchronize(c->done) == hipSuccess && hipFree(c->p) == hipSuccess;
+        c->p = nullptr;
+        if (c->dev != dev) {
+            (void)hipEventDestroy(c->done);
+            c->done = nullptr;
+        }
+    } else if (c->p && c->st != st) {
+        ok = hipStreamWaitEvent(st, c->done, 0) == hipSuccess;
+    }
+    if (ok && !c->done) ok = hipEventCreateWithFlags(&c->done, hipEventDisableTiming) == hipSuccess;
+    if (ok && !c->p) {
+        // some room to grow, within what is kept
+        const size_t nb = bytes > kCutKeep ? bytes : (bytes + bytes / 4 < kCutKeep ? bytes + bytes / 4 : kCutKeep);
+        ok = hipMalloc(&c->p, nb) == hipSuccess;
+        c->bytes = ok ? nb : 0;
+        if (!ok) c->p = nullptr;
+    }
+    if (!ok) {
         (void)hipGetLastError();
         return nullptr;
     }
-    return p;
+    c->dev = dev;
+    c->st = st;
+    c->busy = true;
+    c->used = ++g_cut.clock;
+    return c->p;
 }
 
 void cut_free(void *p, hipStream_t st) {
-    if (p && hipFreeAsync(p, st) != hipSuccess) (void)hipGetLastError();
+    if (!p) return;
+    for (CutBuf &c : g_cut.b) {
+        if (c.p != p) continue;
+        if (c.bytes > kCutKeep || hipEventRecord(c.done, st) != hipSuccess) {
+            (void)hipStreamSynchronize(st);
+            (void)hipFree(c.p);
+            c.p = nullptr;
+            (void)hipGetLastError();
+        }
+        c.busy = false;
+        return;
+    }
 }
 
 }  // namespace bh

@@ -255,8 +255,8 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
             int *flags = (int *)(ws + by + bs);
             T *y = (T *)ws, *snap = (T *)(ws + by);
             cut = SweepCut<T>{g, flags, snap};
-            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, a, lda, n, 0, k + 1, TbMode<MODE>::UPPER ? k : 0,
-                               (int)unit, 5, flags, 0);
+            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, a, lda, n,
+                               CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, flags);
             hipLaunchKernelGGL(kern, dim3(nrhs, g.p), dim3(64), 0, st, n, k, a, lda, (const T *)x, incx, ldx, y, 1,
                                (i64)n, (int)unit, cut);
             hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, nrhs), dim3(64), 0, st, (const T *)snap, CNT, flags);

@@ -150,3 +150,60 @@ def test_cholesky(bh, monkeypatch, dtype, uplo, ldl, kind, n, kd):
         return x.numpy(), info.value
 
     _same(*_both(monkeypatch, run))
+
+
+def _swapped(rng, n, kl, ku, dtype):
+    """Dominant rows 2i and 2i+1 exchanged: half the steps interchange, and the factors are dominant."""
+    A = band(rng, kl - 1, ku - 1, n, np.float64, dist="n")
+    A[ku - 1] += 2 * (kl + ku) + 2
+    B = np.zeros((kl + ku + 1, n))
+    for r in range(kl + ku - 1):  # entry (i, j), i = j + r - (ku - 1), moves to row i ^ 1
+        i = np.arange(n) + r - (ku - 1)
+        to = np.where((i | 1) < n, i ^ 1, i)
+        ok = (i >= 0) & (i < n)
+        B[(ku + to - np.arange(n))[ok], np.arange(n)[ok]] = A[r, ok]
+    return np.asfortranarray(B.astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("kind", ["dominant", "swapped", "random", "nan"])
+@pytest.mark.parametrize("n,kl,ku,nrhs", [
+    (2000, 1, 1, 1), (4097, 4, 4, 3), (20001, 8, 3, 1), (20000, 3, 9, 2), (30000, 16, 16, 1), (16385, 40, 30, 1),
+    (40000, 128, 128, 1), (6000, 0, 5, 2),
+])
+def test_lu_solve(bh, monkeypatch, dtype, trans, kind, n, kl, ku, nrhs):
+    if kind in ("swapped", "nan") and kl == 0:
+        pytest.skip("no interchanges")
+    print(f"gbtrs {dtype.__name__} {trans} {kind} n={n} ({kl},{ku}) nrhs={nrhs}", flush=True)
+    rng = np.random.default_rng(n + kl)
+    A = _swapped(rng, n, kl, ku, dtype) if kind == "swapped" else _system(
+        rng, n, kl, ku, dtype, "random" if kind == "random" else "dominant")
+    F = bh.lu(bh.BandedMatrix.from_host(A, n, kl, ku))
+    if kind == "swapped":
+        assert (F.ipiv != np.arange(1, n + 1)).sum() > n // 3
+    if kind == "nan":
+        f = F.factors.host_data()
+        f[kl + ku + 1, n // 2] = np.nan
+        F.factors.data.upload(f)
+    b = rng.standard_normal((n + 1, nrhs)).astype(dtype)
+    p, t = FP[dtype], trans.encode()
+    args = (n, kl, ku, nrhs, F.factors.data.ptr, F.factors.data.ld, F.ipiv_dev.ptr)
+
+    def run():
+        x = bh.DeviceArray.from_numpy(b)
+        bh._lib.call(f"bh_{p}gbtrs", t, *args, x.ptr, n + 1)
+        return (x.numpy(),)
+
+    on, off = _both(monkeypatch, run)
+    _same(on, off)
+    nb = C.c_size_t(0)
+    bh._lib.call("bh_gbtrs_part_workspace", p.encode(), n, kl, ku, nrhs, C.byref(nb))
+    if nb.value and kind in ("dominant", "swapped"):
+        # the partitioned solve takes the blocks too: then its bits are the exact solve's
+        monkeypatch.delenv("BANDEDHIP_CUT", raising=False)
+        ws, x = bh.DeviceArray((nb.value,), np.uint8), bh.DeviceArray.from_numpy(b)
+        bh._lib.call(f"bh_{p}gbtrs_part", t, *args, x.ptr, n + 1, ws.ptr, nb.value)
+        got, eps = x.numpy().astype(np.float64), np.finfo(dtype).eps
+        # (and where the blocks were refused, rounding: the triangles' condition is under 10 at this dominance)
+        assert np.abs(got - off[0]).max() <= 100 * (kl + ku + 1) * eps * np.abs(off[0]).max()
