@@ -32,9 +32,15 @@
 // not bit for bit: this solve serves the mixed-precision refinement, whose
 // corrections need an accurate solve, not LAPACK's operation order;
 // bh_?gbtrs stays the bit-exact path.
+//
+// Cut systems (bh_cut.hpp).  Where the factors are dominant each sweep runs by
+// blocks of panels, one workgroup per block and 16 right-hand sides, B -> Y
+// -> Z; the LDS window a block leaves must equal, bit for bit, the one the
+// next block has when its own panels begin.
 #include <type_traits>
 
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 #include "bh_mfma.hpp"
 
 namespace bh {
@@ -79,6 +85,8 @@ struct TrsLayout {
         return L;
     }
 };
+
+constexpr int kTrsTrip = 6;  // panels per trip of the sweeps' loops
 
 // ---------------------------------------------------------------- pre-pass
 // One workgroup per panel: perm, L11^{-1} and L21 in final row order, U11^{-1},
@@ -264,9 +272,15 @@ __device__ __forceinline__ void bload_vec(__amdgpu_buffer_rsrc_t r, int off, T (
 // B (n x nrhs, ldb) <- L^{-1} P B for the 16 columns starting at 16*blockIdx.x.
 // LDS addresses are precomputed per lane; the window buffer a panel reads
 // (cur) is a compile-time constant of each of the six unrolled panels.
+// By blocks (cut.g.p > 0) it reads B and writes Y (the same array otherwise).
 template <typename T, int PB, int NW, int MT>
-__global__ __launch_bounds__(64 * NW) void trs_fwd(T *B, i64 ldb, int nrhs, TrsLayout<T, PB> L,
-                                                   const unsigned short *idxA, const T *rec) {
+__global__ __launch_bounds__(64 * NW) void trs_fwd(const T *B, i64 ldb, T *Y, i64 ldy, int nrhs, TrsLayout<T, PB> L,
+                                                   const unsigned short *idxA, const T *rec, SweepCut<T> cut) {
+    const int blk = blockIdx.y;
+    if (cut.g.p > 0 ? cut_closed(cut.flags) : (cut.flags && !cut_failed(cut.flags))) return;
+    // panels p0 .. p1-1, its own from pown: multiples of the trip of six
+    const int p0 = cut.g.p > 0 ? kTrsTrip * cut.g.start(blk) : 0, pown = cut.g.p > 0 ? kTrsTrip * cut.g.own(blk) : 0;
+    const int p1 = cut.g.p > 0 ? min(kTrsTrip * cut.g.end(blk), L.np) : L.np;
     using v4 = typename Mf<T>::v4;
     constexpr int SW = TStride<T>::value;
     constexpr int NS = PB / 4;   // K chunks of a panel product
@@ -285,7 +299,9 @@ __global__ __launch_bounds__(64 * NW) void trs_fwd(T *B, i64 ldb, int nrhs, TrsL
     const int fr = tid >> 4, fj = tid & 15;  // PB*16 <= 64*NW threads carry one fresh element
     const int c0 = 16 * blockIdx.x;
     const bool colok = c0 + jc < nrhs;
-    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(B + (i64)c0 * ldb, 0, (int)(16 * ldb * ES),
+    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(B) + (i64)c0 * ldb, 0,
+                                                                        (int)(16 * ldb * ES), kQRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rY = __builtin_amdgcn_make_buffer_rsrc(Y + (i64)c0 * ldy, 0, (int)(16 * ldy * ES),
                                                                         kQRsrcWord3);
     // per-lane byte offsets inside a panel's records
     const int offA = (int)((L.linv_off + ((size_t)min(w, NP - 1) * 64 + lane) * NS) * ES);
@@ -307,7 +323,7 @@ __global__ __launch_bounds__(64 * NW) void trs_fwd(T *B, i64 ldb, int nrhs, TrsL
     int ysto[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-        ysto[v] = (w < NP && colok) ? (jc * (int)ldb + 16 * w + drow<T>(kq, v)) * ES : kQOob;
+        ysto[v] = (w < NP && colok) ? (jc * (int)ldy + 16 * w + drow<T>(kq, v)) * ES : kQOob;
 
     auto issue = [&](int p, Ops &o) {
         const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
@@ -373,27 +389,37 @@ __global__ __launch_bounds__(64 * NW) void trs_fwd(T *B, i64 ldb, int nrhs, TrsL
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * w + drow<T>(kq, v);
-            const int off = (full || j0 + r < n) && ysto[v] != kQOob ? ysto[v] + j0 * ES : kQOob;
-            qbstore<T>(rB, off, y[v]);
+            const int off = (full || j0 + r < n) && p >= pown && ysto[v] != kQOob ? ysto[v] + j0 * ES : kQOob;
+            qbstore<T>(rY, off, y[v]);
         }
         lds_barrier();
     };
 
     Ops S0, S1, S2;
-    issue(0, S0);
-    issue(min(1, np - 1), S1);
-    // window of panel 0 (buffer 0)
+    issue(p0, S0);
+    issue(min(p0 + 1, np - 1), S1);
+    // window of the first panel (buffer 0)
     for (int e = tid; e < (RWP - 1) * 16; e += 64 * NW) {
-        const int r = e >> 4, j = e & 15;
+        const int r = e >> 4, j = e & 15, row = p0 * PB + r;
         *reinterpret_cast<T *>(lds + r * RS + j * ES) =
-            qbload<T>(rB, (r < RW && r < n && c0 + j < nrhs) ? (j * (int)ldb + r) * ES : kQOob);
+            qbload<T>(rB, (r < RW && row < n && c0 + j < nrhs) ? (j * (int)ldb + row) * ES : kQOob);
     }
     lds_barrier();
+    // the window (buffer 0 between trips) for the seam check; rows past RW hold nothing
+    auto keep = [&](int which) {
+        T *d = cut.at(blk, which, RW * 16);
+        for (int e = tid; e < RW * 16; e += 64 * NW)
+            d[e] = *reinterpret_cast<const T *>(lds + (e >> 4) * RS + (e & 15) * ES);
+    };
     // six panels per trip (three operand sets x two window buffers); panels
     // past the last store nothing: their rows are past n
     const std::integral_constant<int, 0> b0;
     const std::integral_constant<int, 1> b1;
-    for (int p = 0; p < np; p += 6) {
+    for (int p = p0; p < p1; p += kTrsTrip) {
+        if (blk > 0 && p == pown) {
+            keep(0);
+            lds_barrier();
+        }
         panel(p, b0, S0, S2);
         panel(p + 1, b1, S1, S0);
         panel(p + 2, b0, S2, S1);
@@ -401,13 +427,21 @@ __global__ __launch_bounds__(64 * NW) void trs_fwd(T *B, i64 ldb, int nrhs, TrsL
         panel(p + 4, b0, S1, S0);
         panel(p + 5, b1, S2, S1);
     }
+    if (blk + 1 < cut.g.p) keep(1);
 }
 
 // ---------------------------------------------------------------- backward sweep
 // B <- U^{-1} B (U: upper band of width kv = kl+ku) for 16 columns; the U
 // operands come from the pre-pass records.
+// By blocks it reads B and writes X (the same array otherwise).
 template <typename T, int PB, int NW, int MT>
-__global__ __launch_bounds__(64 * NW) void trs_bwd(T *B, i64 ldb, int nrhs, TrsLayout<T, PB> L, const T *rec, int RB) {
+__global__ __launch_bounds__(64 * NW) void trs_bwd(const T *B, i64 ldb, T *X, i64 ldx, int nrhs, TrsLayout<T, PB> L,
+                                                   const T *rec, int RB, SweepCut<T> cut) {
+    const int blk = blockIdx.y;
+    if (cut.g.p > 0 ? cut_closed(cut.flags) : (cut.flags && !cut_failed(cut.flags))) return;
+    // panels by their index from the last one: q0 .. q1-1, its own from qown
+    const int q0 = cut.g.p > 0 ? kTrsTrip * cut.g.start(blk) : 0, qown = cut.g.p > 0 ? kTrsTrip * cut.g.own(blk) : 0;
+    const int q1 = cut.g.p > 0 ? min(kTrsTrip * cut.g.end(blk), L.np) : L.np;
     using v4 = typename Mf<T>::v4;
     constexpr int SW = TStride<T>::value;
     constexpr int NS = PB / 4;
@@ -425,7 +459,9 @@ __global__ __launch_bounds__(64 * NW) void trs_bwd(T *B, i64 ldb, int nrhs, TrsL
     const int fr = tid >> 4, fj = tid & 15;
     const int c0 = 16 * blockIdx.x;
     const bool colok = c0 + jc < nrhs;
-    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(B + (i64)c0 * ldb, 0, (int)(16 * ldb * ES),
+    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(B) + (i64)c0 * ldb, 0,
+                                                                        (int)(16 * ldb * ES), kQRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rX = __builtin_amdgcn_make_buffer_rsrc(X + (i64)c0 * ldx, 0, (int)(16 * ldx * ES),
                                                                         kQRsrcWord3);
     const int offA = (int)((L.uinv_off + ((size_t)min(w, NP - 1) * 64 + lane) * NS) * ES);
     int offB[MT];
@@ -440,7 +476,7 @@ __global__ __launch_bounds__(64 * NW) void trs_bwd(T *B, i64 ldb, int nrhs, TrsL
     int xsto[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-        xsto[v] = (w < NP && colok) ? (jc * (int)ldb + 16 * w + drow<T>(kq, v)) * ES : kQOob;
+        xsto[v] = (w < NP && colok) ? (jc * (int)ldx + 16 * w + drow<T>(kq, v)) * ES : kQOob;
 
     auto issue = [&](int p, Ops &o) {
         const int j0 = p * PB;
@@ -492,17 +528,18 @@ __global__ __launch_bounds__(64 * NW) void trs_bwd(T *B, i64 ldb, int nrhs, TrsL
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * w + drow<T>(kq, v);
-            const int off = (full || (j0 + r >= 0 && j0 + r < n)) && xsto[v] != kQOob ? xsto[v] + j0 * ES : kQOob;
-            qbstore<T>(rB, off, x[v]);
+            const int off =
+                (full || (j0 + r >= 0 && j0 + r < n)) && q >= qown && xsto[v] != kQOob ? xsto[v] + j0 * ES : kQOob;
+            qbstore<T>(rX, off, x[v]);
         }
         lds_barrier();
     };
 
     Ops S0, S1, S2;
-    issue(np - 1, S0);
-    issue(max(np - 2, 0), S1);
-    // ring: rows [jl - top, jl + PB) of the last panel (zero past n)
-    const int jl = (np - 1) * PB;
+    issue(np - 1 - q0, S0);
+    issue(max(np - 2 - q0, 0), S1);
+    // ring: rows [jl - top, jl + PB) of the first panel taken (zero past n)
+    const int jl = (np - 1 - q0) * PB;
     for (int e = tid; e < (top + PB) * 16; e += 64 * NW) {
         const int rr = e >> 4, j = e & 15;
         const int row = jl - top + rr;
@@ -512,15 +549,43 @@ __global__ __launch_bounds__(64 * NW) void trs_bwd(T *B, i64 ldb, int nrhs, TrsL
     lds_barrier();
     // panels before the first (at most two) touch only negative rows: their
     // stores are dropped and their ring updates land in throwaway slots
-    for (int q = 0; q < np; q += 3) {
+    // rows [j0 - top, j0 + PB) of panel q for the seam check
+    auto keep = [&](int which, int q) {
+        const int base = (np - 1 - q) * PB - top;
+        T *d = cut.at(blk, which, (top + PB) * 16);
+        for (int e = tid; e < (top + PB) * 16; e += 64 * NW) {
+            const int row = base + (e >> 4);
+            d[e] = row >= 0 ? *reinterpret_cast<const T *>(Yr + (row & msk) * RS + (e & 15) * ES) : T(0);
+        }
+    };
+    for (int q = q0; q < q1; q += 3) {
+        if (blk > 0 && q == qown) {
+            keep(0, q);
+            lds_barrier();
+        }
         panel(q, S0, S2);
         panel(q + 1, S1, S0);
         panel(q + 2, S2, S1);
     }
+    if (blk + 1 < cut.g.p) keep(1, q1);
 }
 
 constexpr int kTrsPB = 32;
 constexpr int kTrsNW = 8;
+
+// Blocks of a sweep with bandwidth k, in trips of six panels: the lead-in of
+// sweep_geom (20 k rows in FP64, 10 k in FP32, and the window itself); at most
+// 512 workgroups over all groups of 16 right-hand sides, and own trips of at
+// least a quarter of the lead-in (every block reads its lead-in's records again).
+template <typename T>
+CutGeom trs_geom(int np, i64 k, i64 groups) {
+    const int rows = kTrsTrip * kTrsPB;
+    const i64 G = cdiv(np, kTrsTrip), W = cdiv((sizeof(T) == 8 ? 20 : 10) * k, rows) + cdiv(k + kTrsPB, rows);
+    const i64 L = imax(cdiv(G, imax(1, 512 / groups)), (W + 3) / 4);
+    CutGeom g{(int)G, (int)L, (int)W, (int)cdiv(G, L)};
+    if (2 * (L + W) > G || groups > 65535 || g.p < 2 || g.p > 65535) g.p = 0;
+    return g;
+}
 
 }  // namespace
 
@@ -584,7 +649,7 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
     const int RWP = 16 * ((L.RW + 15) / 16) + 1;
     const size_t fl = (size_t)(2 * RWP) * SW * sizeof(T);
     const int mtf = (L.KT + kTrsNW - 1) / kTrsNW;
-    void (*kf)(T *, i64, int, Lt, const unsigned short *, const T *) = nullptr;
+    void (*kf)(const T *, i64, T *, i64, int, Lt, const unsigned short *, const T *, SweepCut<T>) = nullptr;
     if constexpr (sizeof(T) == 4) {
         if (mtf > 3) return BH_ERR_WORKSPACE;
         kf = mtf <= 1 ? trs_fwd<T, kTrsPB, kTrsNW, 1>
@@ -595,13 +660,11 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
         kf = trs_fwd<T, kTrsPB, kTrsNW, 1>;
     }
     if (fl > 64 * 1024) BH_HIP(hipFuncSetAttribute((const void *)kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fl));
-    hipLaunchKernelGGL(kf, grid, dim3(64 * kTrsNW), fl, st, B, ldb, (int)nrhs, L, idx, rec);
-    BH_LAUNCH_CHECK();
     int RB = 1;
     while (RB < 16 * L.KTU + 2 * kTrsPB) RB <<= 1;
     const size_t bl = (size_t)RB * SW * sizeof(T);
     const int mtb = (L.KTU + kTrsNW - 1) / kTrsNW;
-    void (*kb)(T *, i64, int, Lt, const T *, int) = nullptr;
+    void (*kb)(const T *, i64, T *, i64, int, Lt, const T *, int, SweepCut<T>) = nullptr;
     if constexpr (sizeof(T) == 4) {
         kb = mtb <= 1 ? trs_bwd<T, kTrsPB, kTrsNW, 1>
            : mtb == 2 ? trs_bwd<T, kTrsPB, kTrsNW, 2>
@@ -612,9 +675,42 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
         kb = mtb <= 1 ? trs_bwd<T, kTrsPB, kTrsNW, 1> : trs_bwd<T, kTrsPB, kTrsNW, 2>;
     }
     if (bl > 64 * 1024) BH_HIP(hipFuncSetAttribute((const void *)kb, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bl));
-    hipLaunchKernelGGL(kb, grid, dim3(64 * kTrsNW), bl, st, B, ldb, (int)nrhs, L, rec, RB);
-    BH_LAUNCH_CHECK();
-    return BH_OK;
+    // By blocks (gate as in bh_gbtrs_ring.hpp), and behind them the whole
+    // sweeps, which do nothing where the blocks agreed.  16 right-hand sides,
+    // n = 65536, (128,128), FP32: 4.2 -> 0.3 ms, bounded by the W + L links of one block.
+    const dim3 block(64 * kTrsNW);
+    const CutGeom gl = trs_geom<T>(L.np, kl, grid.x), gu = trs_geom<T>(L.np, kl + ku, grid.x);
+    SweepCut<T> cut{};
+    char *ws = nullptr;
+    if (gl.p > 0 && gu.p > 0 && 16 * n * (i64)sizeof(T) < kQOob && cut_enabled()) {
+        auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+        const i64 cols = 16 * (i64)grid.x;  // whole groups of 16 columns
+        const int cl = L.RW * 16, cu = (16 * L.KTU + kTrsPB) * 16;
+        const size_t by = al((size_t)n * cols * sizeof(T)), sl = al((size_t)gl.p * grid.x * 2 * cl * sizeof(T));
+        const size_t su = al((size_t)gu.p * grid.x * 2 * cu * sizeof(T));
+        ws = (char *)cut_alloc(2 * by + sl + su + 256, st);
+        if (ws) {
+            T *Y = (T *)ws, *Z = (T *)(ws + by), *snl = (T *)(ws + 2 * by), *snu = (T *)(ws + 2 * by + sl);
+            int *flags = (int *)(ws + 2 * by + sl + su);
+            const int kd = (int)(kl + ku);
+            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, ab, ldab, (int)n, CutSet{0, kd + 1, kd, 0},
+                               CutSet{kd, (int)kl + 1, kd, 1}, 5, flags);
+            hipLaunchKernelGGL(kf, dim3(grid.x, gl.p), block, fl, st, (const T *)B, ldb, Y, n, (int)nrhs, L, idx, rec,
+                               SweepCut<T>{gl, flags, snl});
+            hipLaunchKernelGGL(sweep_check<T>, dim3(gl.p - 1, grid.x), dim3(64), 0, st, (const T *)snl, cl, flags);
+            hipLaunchKernelGGL(kb, dim3(grid.x, gu.p), block, bl, st, (const T *)Y, n, Z, n, (int)nrhs, L, rec, RB,
+                               SweepCut<T>{gu, flags, snu});
+            hipLaunchKernelGGL(sweep_check<T>, dim3(gu.p - 1, grid.x), dim3(64), 0, st, (const T *)snu, cu, flags);
+            hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n,
+                               (const T *)Z, B, 1, ldb, (const int *)flags);
+            cut.flags = flags;
+        }
+    }
+    hipLaunchKernelGGL(kf, grid, block, fl, st, (const T *)B, ldb, B, ldb, (int)nrhs, L, idx, rec, cut);
+    hipLaunchKernelGGL(kb, grid, block, bl, st, (const T *)B, ldb, B, ldb, (int)nrhs, L, rec, RB, cut);
+    const hipError_t e = hipGetLastError();
+    cut_free(ws, st);
+    return e == hipSuccess ? BH_OK : hip_fail(e, "gbtrs_blocked", __FILE__, __LINE__);
 }
 
 template size_t trs_blocked_bytes<float>(i64, i64, i64);

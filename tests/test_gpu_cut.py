@@ -207,3 +207,29 @@ def test_lu_solve(bh, monkeypatch, dtype, trans, kind, n, kl, ku, nrhs):
         got, eps = x.numpy().astype(np.float64), np.finfo(dtype).eps
         # (and where the blocks were refused, rounding: the triangles' condition is under 10 at this dominance)
         assert np.abs(got - off[0]).max() <= 100 * (kl + ku + 1) * eps * np.abs(off[0]).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["dominant", "swapped", "random", "nan"])
+@pytest.mark.parametrize("n,kl,ku,nrhs", [(6000, 1, 1, 1), (20001, 16, 20, 16), (30000, 40, 17, 17), (65536, 128, 128, 3)])
+def test_blocked_solve(bh, monkeypatch, dtype, kind, n, kl, ku, nrhs):
+    print(f"gbtrs_blocked {dtype.__name__} {kind} n={n} ({kl},{ku}) nrhs={nrhs}", flush=True)
+    rng = np.random.default_rng(n + kl)
+    A = _swapped(rng, n, kl, ku, dtype) if kind == "swapped" else _system(
+        rng, n, kl, ku, dtype, "random" if kind == "random" else "dominant")
+    F = bh.lu(bh.BandedMatrix.from_host(A, n, kl, ku))
+    if kind == "nan":
+        f = F.factors.host_data()
+        f[kl + ku + 1, n // 2] = np.nan
+        F.factors.data.upload(f)
+    b, p, nb = rng.standard_normal((n + 5, nrhs)).astype(dtype), FP[dtype], C.c_size_t(0)
+    bh._lib.call("bh_gbtrs_blocked_workspace", p.encode(), n, kl, ku, C.byref(nb))
+    ws = bh.DeviceArray((nb.value,), np.uint8)
+
+    def run():
+        x = bh.DeviceArray.from_numpy(b)
+        bh._lib.call(f"bh_{p}gbtrs_blocked", n, kl, ku, nrhs, F.factors.data.ptr, F.factors.data.ld, F.ipiv_dev.ptr,
+                     x.ptr, n + 5, ws.ptr, nb.value)
+        return (x.numpy(),)
+
+    _same(*_both(monkeypatch, run))
