@@ -74,57 +74,52 @@ __device__ __forceinline__ int smax(int a, int b) { return a > b ? a : b; }
 //    has exactly R = KL + 1 rows; the steps are unrolled in blocks of U (a
 //    multiple of R), and row i of step s lives in register (i + s) mod R, so
 //    rows never move between registers;
-//  * pivot: every lane takes max |a| over its column's rows (v_max_f64,
-//    which passes over NaN), the pivot column and its max are broadcast to
-//    scalars, and the first row whose |a| equals the max is found with scalar
-//    integer compares -- the reference IDAMAX choice (first largest; a NaN
-//    is never larger, and a NaN first entry is never beaten, so row 0);
-//  * multipliers are formed from the broadcast column, so every lane holds
-//    them without a second broadcast;
+//  * pivot: every lane finds the first largest |a| of its own column (a NaN is
+//    never larger, and never beaten in row 0: the reference IDAMAX choice);
+//    the row and value of the owner become uniform with one readlane each;
+//  * multipliers: every lane scales its own column by the uniform reciprocal,
+//    the owner's are read into scalar registers, which the updates take as
+//    operands, and stored from the owner's lane;
+//  * addresses: a step's uniform part is the instruction's scalar offset, a
+//    lane's part one 24-bit product;
 //  * memory goes through buffer resources: a lane with nothing to load or
 //    store passes an offset past the end (the hardware returns 0 / drops the
 //    store), so no access sits in a branch and the memory counter waits stay
 //    exact; the incoming row of each step is loaded U steps ahead.
+// What bounds a step is the issue of one wave's instructions (about 6.4 cycles
+// each, measured over both forms of the step): n = 10000, (4,4), FP64 with
+// interchanges, 510 -> 385 ns a step when the multipliers left the LDS
+// permutes, the scalar compares and the 64-bit address products.
 constexpr int kBufWord3 = 0x00020000;  // word 3 of a raw buffer resource (gfx9 family)
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, i64 bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, kBufWord3);
 }
-__device__ __forceinline__ double buf_ld(__amdgpu_buffer_rsrc_t r, int off, double) {
+// off: the lane's byte offset (past the end: nothing moves), uni: a uniform one
+__device__ __forceinline__ double buf_ld(__amdgpu_buffer_rsrc_t r, int off, double, int uni = 0) {
     typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, uni, 0));
 }
-__device__ __forceinline__ float buf_ld(__amdgpu_buffer_rsrc_t r, int off, float) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+__device__ __forceinline__ float buf_ld(__amdgpu_buffer_rsrc_t r, int off, float, int uni = 0) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, uni, 0));
 }
-__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int off, double v) {
+__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int off, double v, int uni = 0) {
     typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r, off, uni, 0);
 }
-__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, 0);
+__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int off, float v, int uni = 0) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, uni, 0);
 }
 __device__ __forceinline__ void buf_st64(__amdgpu_buffer_rsrc_t r, int off, long long v) {
     typedef unsigned v2u __attribute__((ext_vector_type(2)));
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v), r, off, 0, 0);
 }
-// |x| as an unsigned integer (order-preserving for non-NaN values)
-__device__ __forceinline__ unsigned long long abs_bits(double x) {
-    return __builtin_bit_cast(unsigned long long, x) & 0x7fffffffffffffffull;
+// whether a uniform value is not +-0, in scalar integer arithmetic
+__device__ __forceinline__ bool nonzero_bits(double x) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    return (((unsigned)(b >> 32) & 0x7fffffffu) | (unsigned)b) != 0;
 }
-__device__ __forceinline__ unsigned abs_bits(float x) { return __builtin_bit_cast(unsigned, x) & 0x7fffffffu; }
-__device__ __forceinline__ unsigned long long inf_bits(double) { return 0x7ff0000000000000ull; }
-// value of lane l in every lane, into a vector register (ds_bpermute)
-__device__ __forceinline__ float lane_bcast(float v, int l) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(l << 2, __builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double lane_bcast(double v, int l) {
-    const long long x = __builtin_bit_cast(long long, v);
-    const int lo = __builtin_amdgcn_ds_bpermute(l << 2, (int)x), hi = __builtin_amdgcn_ds_bpermute(l << 2, (int)(x >> 32));
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ unsigned inf_bits(float) { return 0x7f800000u; }
-
+__device__ __forceinline__ bool nonzero_bits(float x) { return (__builtin_bit_cast(unsigned, x) & 0x7fffffffu) != 0; }
 template <typename T, int KL, bool SOLVE, int UMIN>
 __device__ __forceinline__ int lane_gbsv_wave(int m, int n, int ku, T *__restrict__ ab, i64 ld, i64 *__restrict__ ipiv,
                               T *__restrict__ b) {
@@ -169,12 +164,19 @@ __device__ __forceinline__ int lane_gbsv_wave(int m, int n, int ku, T *__restric
             bpre[s] = buf_ld(rb, off_bin(s), T());
         });
     }
+    // Strides of a step's addresses: with d = (lane - j) mod 64 the lane's
+    // column is j + d, and row j of it lies (j*ld + kv) + d*(ld - 1) elements
+    // into AB: a uniform part (the instruction's scalar offset) and one
+    // 24-bit product.
+    const int dstep = (int)(ld - 1) * SZ, ldb = (int)ld * SZ, kvb = kv * SZ;
+    const int lane0 = lane == 0 ? 0 : -1;  // stores of one uniform value
     // A lane takes column j+64 when column j retires; rows of column j it still
     // holds when j+64 enters the window must read as zero.  Outside the
     // window a lane's rows never move, so one is replaced by an incoming row
     // per step, all of them before j+64 enters unless 2*KL + ku > 63.
     const bool clear_retired = 2 * KL + ku > 63;
     int ju = 0, info = 0, j0 = 0;
+    int ip = 0;  // pivots of the current U steps, step s in lane s
 
     auto step = [&](auto sc, auto tc) {
         constexpr int s = decltype(sc)::value;
@@ -184,126 +186,107 @@ __device__ __forceinline__ int lane_gbsv_wave(int m, int n, int ku, T *__restric
         const int own = j & 63;
         const int km = TAIL ? smin(KL, m - 1 - j) : KL;
         auto reg = [](int i) { return (i + s) % R; };
-        // pivot: max |a| of the lane's column rows 0..km, then the first row of
-        // column j whose |a| equals column j's max
-        T mx = dabs(y[reg(0)]);
+        // pivot: the first row of the largest |a|, found by every lane for its
+        // own column (a NaN is never larger, and never beaten in row 0); the
+        // owner's row and value become uniform
+        T bv = y[reg(0)];
+        int jpl = 0;
 #pragma unroll
-        for (int i = 1; i < R; ++i)
-            if (!TAIL || i <= km) mx = __builtin_fmax(mx, dabs(y[reg(i)]));
-        int jp = 0;
-        T pv;
-        T l[R];
-        bool nz;
-        if constexpr (R <= 3) {
-            // narrow windows: column j broadcast to scalars, scalar compares
-            T xs[R];
-#pragma unroll
-            for (int i = 0; i < R; ++i) xs[i] = lane_read(y[reg(i)], own);
-            const auto mb = abs_bits(lane_read(mx, own));
-#pragma unroll
-            for (int i = R - 1; i >= 1; --i)
-                if ((!TAIL || i <= km) && abs_bits(xs[i]) == mb) jp = i;
-            // row 0 also when its |a| is NaN: nothing compares greater than it
-            if (abs_bits(xs[0]) == mb || abs_bits(xs[0]) > inf_bits(T())) jp = 0;
-            pv = xs[0];
-#pragma unroll
-            for (int i = 1; i < R; ++i)
-                if (jp == i) pv = xs[i];
-            nz = abs_bits(pv) != 0;  // NaN counts as nonzero, as in LAPACK's test
-            const T rcp = T(1) / pv;
-            // multipliers of the interchanged column: a * (1/pivot)
-#pragma unroll
-            for (int i = 1; i < R; ++i) {
-                const T xp = (jp == i) ? xs[0] : xs[i];
-                l[i] = nz ? xp * rcp : xp;
-            }
-        } else {
-            // wide windows (too many values for scalar registers): every lane
-            // finds the pivot row of its own column and forms its own
-            // multipliers; lane own's are broadcast into vector registers
-            const auto mbl = abs_bits(mx);
-            int jpl = 0;
-#pragma unroll
-            for (int i = R - 1; i >= 1; --i)
-                if ((!TAIL || i <= km) && abs_bits(y[reg(i)]) == mbl) jpl = i;
-            if (abs_bits(y[reg(0)]) == mbl || abs_bits(y[reg(0)]) > inf_bits(T())) jpl = 0;
-            jp = __builtin_amdgcn_readlane(jpl, own);
-            T ysel = y[reg(0)];
-#pragma unroll
-            for (int i = 1; i < R; ++i)
-                if (jp == i) ysel = y[reg(i)];
-            pv = lane_read(ysel, own);
-            nz = abs_bits(pv) != 0;
-            const T rcp = T(1) / pv;
-#pragma unroll
-            for (int i = 1; i < R; ++i) {
-                const T xp = (jp == i) ? y[reg(0)] : y[reg(i)];
-                l[i] = lane_bcast(nz ? xp * rcp : xp, own);
+        for (int i = 1; i < R; ++i) {
+            const bool gt = dabs(y[reg(i)]) > dabs(bv);
+            if (!TAIL || i <= km) {
+                bv = gt ? y[reg(i)] : bv;
+                jpl = gt ? i : jpl;
             }
         }
-        if (nz)
-            ju = smax(ju, smin(j + jp + ku, n - 1));
-        else if (info == 0)
-            info = j + 1;
+        const int jp = __builtin_amdgcn_readlane(jpl, own);
+        const T pv = lane_read(bv, own);
+        const bool nz = nonzero_bits(pv);  // NaN counts as nonzero, as in LAPACK's test
+        const int juj = smin(j + jp + ku, n - 1);
+        ju = nz && juj > ju ? juj : ju;
+        info = !nz && info == 0 ? j + 1 : info;
         // interchange rows 0 and jp over columns j..ju only: a lane outside
         // them keeps its rows in place, so the rows a retired column leaves
-        // behind are overwritten by incoming rows within R steps
-        const int c = j + ((lane - j) & 63);
-        if (jp != 0 && c <= ju) {
+        // behind are overwritten by incoming rows within R steps.  (Selects on
+        // scalar conditions: a chain of branches costs copies of every row
+        // where they join.)
+        const int d = (lane - j) & 63;
+        if (jp != 0) {
+            const bool live = d <= ju - j;
+            const T t0 = y[reg(0)], b0 = SOLVE ? bw[reg(0)] : T(0);
+            T t = t0, b1 = b0;
 #pragma unroll
-            for (int i = 1; i < R; ++i)
-                if (jp == i) {
-                    const T t0 = y[reg(0)];
-                    y[reg(0)] = y[reg(i)];
-                    y[reg(i)] = t0;
+            for (int i = 1; i < R; ++i) {
+                const bool sw = (jp == i) & live;
+                t = sw ? y[reg(i)] : t;
+                y[reg(i)] = sw ? t0 : y[reg(i)];
+                if (SOLVE) {
+                    b1 = jp == i ? bw[reg(i)] : b1;
+                    bw[reg(i)] = jp == i ? b0 : bw[reg(i)];
                 }
+            }
+            y[reg(0)] = t;
+            if (SOLVE) bw[reg(0)] = b1;
         }
-        // rank-1 update of columns j+1..ju, rows 1..km
-        if (nz && c > j && c <= ju) {
+        // multipliers: every lane scales its own column; lane own's are read
+        // into scalar registers, which the updates take as operands
+        const T rcp = nz ? T(1) / pv : T(1);
+        T lc[R], l[R];
+#pragma unroll
+        for (int i = 1; i < R; ++i) {
+            lc[i] = y[reg(i)] * rcp;
+            l[i] = lane_read(lc[i], own);
+        }
+        // U row j (lanes of columns j..j+kv; the pivot from lane own), then
+        // column j's multipliers from lane own
+        const int rowb = j * ldb + kvb;
+        buf_st(rab, d <= smin(kv, n - 1 - j) ? (int)__umul24(d, dstep) : -1, y[reg(0)], rowb);
+        const int vown = d == 0 ? 0 : -(1 << 30);
+#pragma unroll
+        for (int i = 1; i < R; ++i)
+            if (!TAIL || i <= km) buf_st(rab, vown + i * SZ, lc[i], rowb);
+        ip = lane == s ? j + jp + 1 : ip;
+        // rank-1 update of columns j+1..ju, rows 1..km (a zero pivot updates nothing)
+        if ((unsigned)(d - 1) < (unsigned)(nz ? ju - j : 0)) {
             const T nu = -y[reg(0)];
 #pragma unroll
             for (int i = 1; i < R; ++i)
                 if (!TAIL || i <= km) y[reg(i)] = dfma(l[i], nu, y[reg(i)]);
         }
-        // U row j (lanes of columns j..j+kv; the pivot from lane own), then
-        // column j's multipliers and the pivot index
-        buf_st(rab, (c - j <= kv && c < n) ? (int)(((i64)c * ld + kv - (c - j)) * SZ) : -1, y[reg(0)]);
-#pragma unroll
-        for (int i = 1; i < R; ++i)
-            if (!TAIL || i <= km) buf_st(rab, lane == 0 ? (int)(((i64)j * ld + kv + i) * SZ) : -1, l[i]);
-        buf_st64(rip, lane == 0 ? j * 8 : -1, (long long)(j + jp + 1));
         if (SOLVE) {
             // forward substitution step j (xGBTRS: interchange, then the L column)
-            if (jp != 0) {
-#pragma unroll
-                for (int i = 1; i < R; ++i)
-                    if (jp == i) {
-                        const T t0 = bw[reg(0)];
-                        bw[reg(0)] = bw[reg(i)];
-                        bw[reg(i)] = t0;
-                    }
-            }
             const T nb = -bw[reg(0)];
             const int kb = TAIL ? smin(KL, n - 1 - j) : KL;
 #pragma unroll
             for (int i = 1; i < R; ++i)
                 if (!TAIL || i <= kb) bw[reg(i)] = dfma(l[i], nb, bw[reg(i)]);
-            buf_st(rb, lane == 0 ? j * SZ : -1, bw[reg(0)]);
+            buf_st(rb, lane0, bw[reg(0)], j * SZ);
             bw[reg(0)] = bpre[s];
             bpre[s] = buf_ld(rb, off_bin(j + U), T());
         }
-        if (clear_retired && lane == own) {
+        if (clear_retired && d == 0) {
 #pragma unroll
-            for (int i = 0; i < R; ++i) y[i] = T(0);
+            for (int i = 1; i < R; ++i) y[reg(i)] = T(0);
         }
         y[reg(0)] = pre[s];
-        pre[s] = buf_ld(rab, off_in(j + U), T());
+        {
+            const int J = j + U + 1, dj = (lane - J) & 63;  // the row entering at the end of step j+U
+            const int lim = (J <= mn && J + KL < m) ? smin(kv, n - 1 - J) : -1;
+            pre[s] = buf_ld(rab, dj <= lim ? (int)__umul24(dj, dstep) : -1, T(), J * ldb + kvb + KL * SZ);
+        }
+    };
+    auto put_pivots = [&] {
+        buf_st64(rip, (lane < U && j0 + lane < mn) ? (j0 + lane) * 8 : -1, (long long)ip);
     };
     const int jmain = smin(mn, m - KL);  // steps before it have km == KL
-    for (; j0 + U <= jmain; j0 += U)
+    for (; j0 + U <= jmain; j0 += U) {
         SUnroll<U>::run([&](auto sc) { step(sc, std::false_type{}); });
-    for (; j0 < mn; j0 += U)
+        put_pivots();
+    }
+    for (; j0 < mn; j0 += U) {
         SUnroll<U>::run([&](auto sc) { step(sc, std::true_type{}); });
+        put_pivots();
+    }
 
     // Fill-in rows LAPACK zeroes that no U row covered (rows >= m).
     {
@@ -431,7 +414,9 @@ int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64
                       const LuCut<BH_LANE_T> *cut) {
     using T = BH_LANE_T;
     const i64 nb = cut && cut->g.p > 0 ? cut->g.span() : n;  // a block's copy holds span() columns
-    if (kl + ku > 63 || m >= (1ll << 30) || n >= (1ll << 30) || ldab * nb * (i64)sizeof(T) >= (1ll << 31)) return -1;
+    if (kl + ku > 63 || m >= (1ll << 30) || n >= (1ll << 30) || ldab * nb * (i64)sizeof(T) >= (1ll << 31) ||
+        ldab * (i64)sizeof(T) >= (1ll << 24))
+        return -1;
     const int mi = (int)m, ni = (int)n, ui = (int)ku;
     const LuCut<T> c = cut ? *cut : LuCut<T>{};
     const dim3 grid(c.g.p > 0 ? (unsigned)c.g.p : 1u);
