@@ -14,6 +14,8 @@
 // In this file u is the padded upper bandwidth u' (the storage's own).
 //
 // Kernels:
+//   * gbqrf_lane, qtb_lane (bh_gbqr_lane.hpp): l <= 7, the narrow bands' own
+//     kernels with the same arithmetic.
 //   * gbqrf_wave: one wave per system.  Lane c holds band column c of the
 //     live window (columns k .. k+u, lane = column mod 64) with its rows
 //     k .. k+l in registers; every lane computes the step-k reflector from
@@ -38,6 +40,7 @@
 // band solve of R (tribanded.jl:75-83 -> tbsv), which is the back
 // substitution of the band LU solve with no L part.
 #include "bh_common.hpp"
+#include "bh_gbqr_lane.hpp"
 
 namespace bh {
 
@@ -507,6 +510,10 @@ int gbqrf_impl(i64 m, i64 n, i64 l, i64 u, T *D, i64 ldd, T *tau) {
     if (m == 0 || n == 0) return BH_OK;
     hipStream_t st = stream();
     const int mi = (int)m, ni = (int)n, li = (int)l, ui = (int)u;
+    {
+        const int r = lane_gbqrf_launch(m, n, l, u, D, ldd, tau, st);
+        if (r != -1) return r;
+    }
 #define BH_QR_CASE(RLv)                                                                      \
     if (l + 1 <= RLv && u + 1 <= 64) {                                                       \
         hipLaunchKernelGGL((gbqrf_wave<T, RLv>), dim3(1), dim3(64), 0, st, mi, ni, li, ui, D, ldd, tau); \
@@ -548,6 +555,10 @@ int gbqrm_impl(char trans, i64 m, i64 n, i64 l, i64 u, const T *D, i64 ldd, cons
     const bool tr = !(trans == 'N' || trans == 'n');
     const int kmax = (int)imin(m, n);
     hipStream_t st = stream();
+    if (tr) {
+        const int r = lane_qtb_launch(m, n, l, u, D, ldd, tau, nrhs, B, ldb, st);
+        if (r != -1) return r;
+    }
     if (l + 1 <= 64) {
         hipLaunchKernelGGL(gbqr_apply_wave<T>, dim3((unsigned)nrhs), dim3(64), 0, st, tr, (int)m, (int)n, (int)l,
                            (int)u, D, ldd, tau, kmax, B, ldb);
