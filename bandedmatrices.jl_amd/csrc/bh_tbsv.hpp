@@ -4,6 +4,7 @@
 #pragma once
 #include "bh_common.hpp"
 #include "bh_cut.hpp"
+#include "bh_tbsv_lane.hpp"
 
 namespace bh {
 
@@ -238,8 +239,8 @@ __global__ void __launch_bounds__(kTbBlock) tbsv_block(int n, int k, const T *__
 // The ring solve: by blocks where the triangle's columns are dominated by
 // their diagonal (1.25 times the rest, or 1 for a unit diagonal), and behind
 // them the whole sweep, which does nothing where the blocks agreed.  Measured
-// 'N' upper FP64: n = 2^20, k = 8 143 -> 0.35 ms (what bounds it: 0.14 us a step
-// over a block's steps, then the launches); a triangle that fails the gate pays the gate
+// 'N' upper FP64: n = 2^20, k = 8 143 -> 0.31 ms by rings, 0.156 by lanes (rings: 0.3 us a step
+// over a block's steps with two waves to a SIMD); a triangle that fails the gate pays the gate
 // and four empty launches, about 25 us.
 template <typename T, int MODE, int NW, int PFD>
 int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx, int nrhs, bool unit, hipStream_t st) {
@@ -248,20 +249,36 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
     SweepCut<T> cut{};
     char *ws = nullptr;
     const CutGeom g = sweep_geom<T>(n, k, nrhs, NW);
-    if (g.p > 0 && cut_enabled()) {
-        const size_t by = ((size_t)n * nrhs * sizeof(T) + 255) & ~(size_t)255, bs = (size_t)g.p * nrhs * 2 * CNT * sizeof(T);
+    // 'N' with k <= 16: one lane per block (bh_tbsv_lane.hpp), where the blocks
+    // are the shorter (L + W steps of 0.1-0.2 us against 0.3)
+    TbsvLane gl;
+    if (TbMode<MODE>::AXPY) gl = tbsv_lane_geom(n, k, lda, incx, ldx, nrhs, (int)sizeof(T));
+    if ((gl.p > 0 || g.p > 0) && cut_enabled()) {
+        const size_t by = ((size_t)n * nrhs * sizeof(T) + 255) & ~(size_t)255;
+        const size_t bs = gl.p > 0 ? (tbsv_lane_bytes(gl, k, nrhs, sizeof(T)) + 255) & ~(size_t)255
+                                   : (size_t)g.p * nrhs * 2 * CNT * sizeof(T);
         ws = (char *)cut_alloc(by + bs + 256, st);
         if (ws) {
             int *flags = (int *)(ws + by + bs);
             T *y = (T *)ws, *snap = (T *)(ws + by);
-            cut = SweepCut<T>{g, flags, snap};
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, a, lda, n,
                                CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, flags);
-            hipLaunchKernelGGL(kern, dim3(nrhs, g.p), dim3(64), 0, st, n, k, a, lda, (const T *)x, incx, ldx, y, 1,
-                               (i64)n, (int)unit, cut);
-            hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, nrhs), dim3(64), 0, st, (const T *)snap, CNT, flags);
+            if (gl.p > 0) {
+                const int r = tbsv_lane_run(gl, TbMode<MODE>::ASC, n, k, a, lda, x, incx, ldx, nrhs, unit, y, snap,
+                                            flags, st);
+                if (r != BH_OK) {
+                    cut_free(ws, st);
+                    return r;
+                }
+            } else {
+                cut = SweepCut<T>{g, flags, snap};
+                hipLaunchKernelGGL(kern, dim3(nrhs, g.p), dim3(64), 0, st, n, k, a, lda, (const T *)x, incx, ldx, y, 1,
+                                   (i64)n, (int)unit, cut);
+                hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, nrhs), dim3(256), 0, st, (const T *)snap, CNT, flags);
+            }
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), nrhs), dim3(256), 0, st, n, (const T *)y,
                                x, incx, ldx, (const int *)flags);
+            cut.flags = flags;
             cut.g.p = 0;
         }
     }
