@@ -85,32 +85,38 @@ struct LuCut {
     }
 };
 
-// Gate: 256 columns spread over the matrix, 16 lanes to a column; closed when
-// more than a quarter of them have num/4 times the sum of |a| off the
+// The blocks of a one-lane-per-block Cholesky (bh_pbtrf_lane.hip).
+struct PbLane {
+    int p, L, W;  // blocks, own columns, lead-in
+};
+
+// Gate: 256 columns spread over the matrix, 16 lanes to a column (64 columns
+// and a wave to each where they are longer than 64 entries: 42 -> 19 us at
+// 385 and 129 entries); closed when more than a quarter of them have num/4 times the sum of |a| off the
 // diagonal above |a_jj|.  One workgroup, so it writes both flags itself.
 // A set of entries of a column: rows r0 .. r0+h-1 of the band array, the
 // diagonal in row d (with `unit` it counts as 1); h = 0: no second set.
 struct CutSet {
     int r0, h, d, unit;
 };
-constexpr int kCutSamples = 256;
 template <typename T>
 __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, CutSet s1, CutSet s2, int num,
                                                  int *flags) {
     __shared__ int weak[2];
     if (threadIdx.x < 2) weak[threadIdx.x] = 0;
     __syncthreads();
-    const int g = threadIdx.x >> 4, q = threadIdx.x & 15;
+    const int lanes = s1.h > 64 ? 64 : 16, cols = 1024 / lanes, samples = 4 * cols;
+    const int g = threadIdx.x / lanes, q = threadIdx.x & (lanes - 1);
     int m1 = 0, m2 = 0;
     auto strong = [&](const T *col, const CutSet &s) {
         T t = T(0);
-        for (int r = q; r < s.h; r += 16) t += (s.r0 + r == s.d) ? T(0) : dabs(col[s.r0 + r]);
-        for (int off = 8; off > 0; off >>= 1) t += __shfl_xor(t, off, 16);
+        for (int r = q; r < s.h; r += lanes) t += (s.r0 + r == s.d) ? T(0) : dabs(col[s.r0 + r]);
+        for (int off = lanes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
         return T(4) * (s.unit ? T(1) : dabs(col[s.d])) >= T(num) * t;
     };
 #pragma unroll
-    for (int it = 0; it < kCutSamples / 64; ++it) {
-        const i64 c = ((i64)(64 * it + g) * n + n / 2) / kCutSamples;
+    for (int it = 0; it < 4; ++it) {
+        const i64 c = ((i64)(cols * it + g) * n + n / 2) / samples;
         const T *col = a + c * ld;
         m1 += !strong(col, s1);
         if (s2.h) m2 += !strong(col, s2);
@@ -121,7 +127,7 @@ __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        flags[0] = weak[0] > kCutSamples / 4 || weak[1] > kCutSamples / 4;
+        flags[0] = weak[0] > samples / 4 || weak[1] > samples / 4;
         flags[1] = 0;
     }
 }
@@ -150,13 +156,14 @@ struct RingCutWs {
 
 // cnt entries per window; grid (p - 1, nrhs)
 template <typename T>
-__global__ void __launch_bounds__(64) sweep_check(const T *__restrict__ snap, int cnt, int *flags) {
+__global__ void __launch_bounds__(256) sweep_check(const T *__restrict__ snap, int cnt, int *flags) {
     if (cut_closed(flags)) return;
     const T *e = snap + (((i64)blockIdx.x * gridDim.y + blockIdx.y) * 2 + 1) * cnt;
     const T *s = snap + (((i64)(blockIdx.x + 1) * gridDim.y + blockIdx.y) * 2) * cnt;
     bool bad = false;
-    for (int i = threadIdx.x; i < cnt; i += 64) bad |= cut_differ(e[i], s[i]);
-    if (__any(bad) && threadIdx.x == 0) atomicOr(flags + 1, 1);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < cnt; i += 256) bad |= cut_differ(e[i], s[i]);
+    if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(flags + 1, 1);
 }
 
 // the blocks' results (n x nrhs, contiguous) to the caller's vectors

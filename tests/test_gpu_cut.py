@@ -233,3 +233,27 @@ def test_blocked_solve(bh, monkeypatch, dtype, kind, n, kl, ku, nrhs):
         return (x.numpy(),)
 
     _same(*_both(monkeypatch, run))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kd", range(1, 10))
+def test_cholesky_narrow(bh, monkeypatch, dtype, kd):
+    """Every width of the one-lane-per-block kernel and one more, at lengths around its blocks; NaN in the unused corner."""
+    for n in (600, 601, 1999, 8192, 20011):
+        print(f"cholesky {dtype.__name__} n={n} kd={kd}", flush=True)
+        rng = np.random.default_rng(n + kd)
+        A = rng.uniform(-1, 1, (kd + 1, n))
+        A[kd] = kd + 2 + rng.random(n)
+        A[0, n // 2] = -0.0
+        for c in range(kd):
+            A[: kd - c, c] = np.nan
+        ab = np.asfortranarray(A.astype(dtype))
+
+        def run():
+            x, info = bh.DeviceArray.from_numpy(ab), C.c_int64(-7)
+            bh._lib.call(f"bh_{FP[dtype]}pbtrf", b"U", n, kd, x.ptr, kd + 1, C.byref(info))
+            return x.numpy(), info.value
+
+        on, off = _both(monkeypatch, run)
+        assert off[1] == 0
+        _same(on, off)
