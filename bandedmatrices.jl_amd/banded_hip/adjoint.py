@@ -9,7 +9,7 @@ P restricts an outer product to A's band (band storage, like A.data).
 """
 from __future__ import annotations
 
-import numpy as np
+import ctypes as C
 
 from . import _lib
 from .bandedmatrix import BandedMatrix, _prefix, mul
@@ -63,6 +63,6 @@ def loss_and_grad(A: BandedMatrix, b: DeviceArray, w: DeviceArray, x0: DeviceArr
     dA = BandedMatrix.zeros((n, n), A.bandwidths(), A.dtype)
     _lib.call(f"bh_{_prefix(A.dtype)}gb_band_grad", n, n, A.l, A.u, lam.ptr, x.ptr, y0.ptr, x0.ptr, dA.data.ptr,
               dA.data.ld)
-    xh, wh, yh = x.numpy(), w.numpy(), y0.numpy()
-    L = float(np.dot(wh, xh) + 0.5 * np.dot(yh, yh))
-    return L, dA, lam, x
+    L = C.c_double(0.0)
+    _lib.call(f"bh_{_prefix(A.dtype)}gb_loss", n, w.ptr, x.ptr, y0.ptr, C.byref(L))
+    return L.value, dA, lam, x

@@ -196,10 +196,11 @@ __global__ void __launch_bounds__(256) lu_cut_check(LuCut<T> cut, int kv, int cm
     if (cut.g.start(blk) > 0) {
         const int c0 = cut.g.own(blk) - cmp, a0 = c0 - cut.g.start(blk - 1), b0 = c0 - cut.g.start(blk);
         const T *a = cut.block_ab(blk - 1), *b = cut.block_ab(blk);
-        for (int e = threadIdx.x; e < cmp * cut.kl; e += 256) {
-            const int c = e / cut.kl, r = kv + 1 + e - c * cut.kl;
-            bad |= cut_differ(a[(i64)(a0 + c) * H + r], b[(i64)(b0 + c) * H + r]);
-        }
+        // a wave to a column, four columns in flight
+#pragma unroll 4
+        for (int c = threadIdx.x >> 6; c < cmp; c += 4)
+            for (int r = kv + 1 + (threadIdx.x & 63); r <= kv + cut.kl; r += 64)
+                bad |= cut_differ(a[(i64)(a0 + c) * H + r], b[(i64)(b0 + c) * H + r]);
         const i64 *pa = cut.ipiv + (i64)(blk - 1) * cut.g.span(), *pb = cut.ipiv + (i64)blk * cut.g.span();
         for (int c = threadIdx.x; c < cmp; c += 256) bad |= pa[a0 + c] - a0 != pb[b0 + c] - b0;
     }

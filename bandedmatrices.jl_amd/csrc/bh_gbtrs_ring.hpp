@@ -451,7 +451,7 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
                 T *snap = lower ? snl : snu;
                 hipLaunchKernelGGL(kern, dim3((unsigned)nrhs, g.p), block, 0, st, (int)n, (int)kl, (int)ku, ab, ld, ipiv,
                                    RingWork<T>{sweep, in, out, ldin, n, SweepCut<T>{g, flags, snap}});
-                hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, (unsigned)nrhs), block, 0, st, (const T *)snap,
+                hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, (unsigned)nrhs), dim3(256), 0, st, (const T *)snap,
                                    64 * (lower ? NF : NB), flags);
                 in = out;
                 ldin = n;

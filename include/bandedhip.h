@@ -367,6 +367,10 @@ int bh_dgb_band_grad(bh_int m, bh_int n, bh_int kl, bh_int ku, const double *lam
                      const double *y0, const double *x0, double *G, bh_int ldg);
 int bh_sgb_band_grad(bh_int m, bh_int n, bh_int kl, bh_int ku, const float *lam, const float *x,
                      const float *y0, const float *x0, float *G, bh_int ldg);
+/* That loss itself, *loss_host = w'x + 1/2 y'y over n entries, summed on the
+ * device in double in a fixed order; waits for the stream. */
+int bh_dgb_loss(bh_int n, const double *w, const double *x, const double *y, double *loss_host);
+int bh_sgb_loss(bh_int n, const float *w, const float *x, const float *y, double *loss_host);
 /* G <- beta G + P(alpha1 u1 v1' + alpha2 u2 v2'), P = restriction to the band,
  * each term one fma(alpha u_i, v_j, g) in that order; a NULL (u, v) pair is
  * skipped.  The pullbacks of A \ b (alpha = -1, u = A^{-T} xbar, v = x) and of
