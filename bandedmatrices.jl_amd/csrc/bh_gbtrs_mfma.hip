@@ -103,17 +103,14 @@ __global__ __launch_bounds__(256) void trs_prep(const T *__restrict__ ab, i64 ld
     T *Lf = reinterpret_cast<T *>(tp_raw);  // RW x LS
     T *Ut = Lf + (size_t)RW * LS;           // PB x LS
     T *Xi = Ut + PB * LS;                   // PB x LS
-    T *Ub = Xi + PB * LS;                   // top x LS: U block above the panel
+    T *Xu = Xi + PB * LS;                   // PB x LS
+    T *Ub = Xu + PB * LS;                   // top x LS: U block above the panel
     int *perm = reinterpret_cast<int *>(Ub + (size_t)top * LS);
-    int *F = perm + RW;
     __shared__ int q[PB];
     const int p = blockIdx.x, tid = threadIdx.x;
     const int j0 = p * PB, nb = min(PB, n - j0);
     for (int e = tid; e < RW * LS; e += 256) Lf[e] = T(0);
-    for (int r = tid; r < RW; r += 256) {
-        perm[r] = r;
-        F[r] = r;
-    }
+    for (int r = tid; r < RW; r += 256) perm[r] = r;
     if (tid < PB) {
         int qq = tid;
         if (tid < nb) {
@@ -131,19 +128,24 @@ __global__ __launch_bounds__(256) void trs_prep(const T *__restrict__ ab, i64 ld
         }
     }
     // multipliers of column c sit at positions c+1..c+kl after step c; the
-    // later interchanges of the panel carry position r to F_c(r)
-    for (int c = nb - 1; c >= 0; --c) {
-        const i64 col = (i64)(j0 + c) * ldab;
-        for (int r = c + 1 + tid; r <= c + kl && r < RW; r += 256)
-            if (j0 + r < n) Lf[F[r] * LS + c] = ab[col + (kv + r - c)];
-        __syncthreads();
-        if (tid == 0 && q[c] != c) {
-            const int a = F[c];
-            F[c] = F[q[c]];
-            F[q[c]] = a;
+    // later interchanges of the panel carry position r on.  Every thread
+    // follows its own entries through them (with a barrier per column, each
+    // waited for its column's load).  2048 panels, (128,128), FP32: 455 -> 420 us
+    // with that, 257 with the inverses in registers and the products below
+    // eight chunks to a thread.  (U's block read along its columns instead
+    // cost 25 us: its LDS writes then conflict.)
+    const bool moved = __syncthreads_or(tid < PB && q[tid < PB ? tid : 0] != tid);
+    for (int e = tid; e < nb * kl; e += 256) {
+        const int c = e / kl, r = c + 1 + e - c * kl;
+        if (r < RW && j0 + r < n) {
+            const T v = ab[(i64)(j0 + c) * ldab + (kv + r - c)];
+            int f = r;
+            if (moved)
+                for (int s = c + 1; s < nb; ++s) f = f == s ? q[s] : f == q[s] ? s : f;
+            Lf[f * LS + c] = v;
         }
-        __syncthreads();
     }
+    __syncthreads();
     if (tid < PB) Lf[tid * LS + tid] = T(1);
     // U11 (upper, identity past the last column)
     for (int e = tid; e < PB * PB; e += 256) {
@@ -156,17 +158,42 @@ __global__ __launch_bounds__(256) void trs_prep(const T *__restrict__ ab, i64 ld
         Ut[i * LS + j] = v;
     }
     __syncthreads();
-    // L11^{-1}: column j by forward substitution (thread j)
+    // U(i, j) above the panel: i = j0 - top + r, j = j0 + c
+    for (int e = tid; e < top * PB; e += 256) {
+        const int r = e / PB, c = e - r * PB;
+        const int i = j0 - top + r, j = j0 + c, d = kv + i - j;
+        Ub[r * LS + c] = (i >= 0 && j < n && d >= 0) ? ab[(i64)j * ldab + d] : T(0);
+    }
+    // The inverses, one column to a thread, in registers and fully unrolled:
+    // L11^{-1} by forward substitution on the first wave, U11^{-1} by back
+    // substitution on the second.
     if (tid < PB) {
         const int j = tid;
+        T X[PB];
+#pragma unroll
         for (int i = 0; i < PB; ++i) {
-            T x = (i == j) ? T(1) : T(0);
-            if (i > j) {
-                T s = T(0);
-                for (int k = j; k < i; ++k) s = dfma(Lf[i * LS + k], Xi[k * LS + j], s);
-                x = -s;
+            T s = T(0);
+#pragma unroll
+            for (int k = 0; k < i; ++k) {
+                const T f = dfma(Lf[i * LS + k], X[k], s);
+                s = k >= j ? f : s;
             }
-            Xi[i * LS + j] = x;
+            X[i] = i > j ? -s : (i == j ? T(1) : T(0));
+            Xi[i * LS + j] = X[i];
+        }
+    } else if (tid >= 64 && tid < 64 + PB) {
+        const int j = tid - 64;
+        T X[PB];
+#pragma unroll
+        for (int i = PB - 1; i >= 0; --i) {
+            T s = (i == j) ? T(1) : T(0);
+#pragma unroll
+            for (int k = i + 1; k < PB; ++k) {
+                const T f = dfma(-Ut[i * LS + k], X[k], s);
+                s = k <= j ? f : s;
+            }
+            X[i] = i <= j ? s / Ut[i * LS + i] : T(0);
+            Xu[i * LS + j] = X[i];
         }
     }
     __syncthreads();
@@ -175,23 +202,36 @@ __global__ __launch_bounds__(256) void trs_prep(const T *__restrict__ ab, i64 ld
     // element e of a tile block: tile e / (64 NS), lane (e / NS) % 64, chunk e % NS
     for (int e = tid; e < PB * PB; e += 256) {
         const int s = e % NS, lane = (e / NS) & 63, ti = e / (64 * NS);
-        out[L.linv_off + e] = Xi[(16 * ti + (lane & 15)) * LS + 4 * s + (lane >> 4)];
+        const int at = (16 * ti + (lane & 15)) * LS + 4 * s + (lane >> 4);
+        out[L.linv_off + e] = Xi[at];
+        out[L.uinv_off + e] = Xu[at];
     }
-    // -M21 = -L21 L11^{-1} (L11^{-1} lower triangular)
-    for (int e = tid; e < L.KT * 16 * PB; e += 256) {
-        const int s = e % NS, lane = (e / NS) & 63, t = e / (64 * NS);
-        const int r = PB + 16 * t + (lane & 15), c = 4 * s + (lane >> 4);
-        T acc = T(0);
-        if (r < RW)
-            for (int k = c; k < PB; ++k) acc = dfma(Lf[r * LS + k], Xi[k * LS + c], acc);
-        out[L.l21_off + e] = -acc;  // stored negated: the sweep accumulates onto the C operand
-    }
-    // U(i, j) above the panel: i = j0 - top + r, j = j0 + c
-    for (int e = tid; e < top * PB; e += 256) {
-        const int r = e / PB, c = e - r * PB;
-        const int i = j0 - top + r, j = j0 + c, d = kv + i - j;
-        Ub[r * LS + c] = (i >= 0 && j < n && d >= 0) ? ab[(i64)j * ldab + d] : T(0);
-    }
+    // -M21 = -L21 L11^{-1} and -V = -U_block U11^{-1}, stored negated (the sweeps
+    // accumulate onto the C operand): a thread forms the NS chunks of one
+    // lane's row together, the inverse's triangle kept by selects
+    auto product = [&](const T *A, int rows, const T *X, bool low, int tiles, size_t off) {
+        for (int e = tid; e < tiles * 64; e += 256) {
+            const int lane = e & 63, r = 16 * (e >> 6) + (lane & 15), kq = lane >> 4;
+            const T *row = A + min(r, rows - 1) * LS;
+            T acc[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) acc[s] = T(0);
+#pragma unroll 8
+            for (int k = 0; k < PB; ++k) {
+                const T a = row[k];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const int c = 4 * s + kq;
+                    const T f = dfma(a, X[k * LS + c], acc[s]);
+                    acc[s] = (low ? k >= c : k <= c) ? f : acc[s];
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s) out[off + (size_t)e * NS + s] = r < rows ? -acc[s] : -T(0);
+        }
+    };
+    product(Lf + PB * LS, RW - PB, Xi, true, L.KT, L.l21_off);
+    product(Ub, top, Xu, false, L.KTU, L.ublk_off);
     unsigned short *ix = idxA + (size_t)p * L.idx_u16;
     // window rows as LDS byte offsets of the sweep's [rows][SW] buffer (< 2^16)
     constexpr int RB_ = TStride<T>::value * (int)sizeof(T);
@@ -199,33 +239,6 @@ __global__ __launch_bounds__(256) void trs_prep(const T *__restrict__ ab, i64 ld
     for (int e = tid; e < L.KT * 16; e += 256) {
         const int v = e & 3, kq = (e >> 2) & 3, t = e >> 4;
         ix[L.cidx_off + e] = (unsigned short)(perm[min(PB + 16 * t + drow<T>(kq, v), RW - 1)] * RB_);
-    }
-    __syncthreads();
-    // U11^{-1}: column j by back substitution (thread j)
-    if (tid < PB) {
-        const int j = tid;
-        for (int i = PB - 1; i >= 0; --i) {
-            T x = T(0);
-            if (i <= j) {
-                T s = (i == j) ? T(1) : T(0);
-                for (int k = i + 1; k <= j; ++k) s = dfma(-Ut[i * LS + k], Xi[k * LS + j], s);
-                x = s / Ut[i * LS + i];
-            }
-            Xi[i * LS + j] = x;
-        }
-    }
-    __syncthreads();
-    for (int e = tid; e < PB * PB; e += 256) {
-        const int s = e % NS, lane = (e / NS) & 63, ti = e / (64 * NS);
-        out[L.uinv_off + e] = Xi[(16 * ti + (lane & 15)) * LS + 4 * s + (lane >> 4)];
-    }
-    // V = U_block U11^{-1} (U11^{-1} upper triangular), stored negated
-    for (int e = tid; e < L.KTU * 16 * PB; e += 256) {
-        const int s = e % NS, lane = (e / NS) & 63, t = e / (64 * NS);
-        const int r = 16 * t + (lane & 15), c = 4 * s + (lane >> 4);
-        T acc = T(0);
-        for (int k = 0; k <= c; ++k) acc = dfma(Ub[r * LS + k], Xi[k * LS + c], acc);
-        out[L.ublk_off + e] = -acc;
     }
 }
 
@@ -607,7 +620,7 @@ size_t trs_blocked_bytes(i64 n, i64 kl, i64 ku) {
     int RB = 1;
     while (RB < 16 * L.KTU + 2 * kTrsPB) RB <<= 1;
     const size_t bwd_lds = (size_t)RB * SW * sizeof(T);
-    const size_t prep_lds = ((size_t)(L.RW + 2 * kTrsPB + 16 * L.KTU) * (kTrsPB + 1)) * sizeof(T) + 2 * L.RW * sizeof(int);
+    const size_t prep_lds = ((size_t)(L.RW + 3 * kTrsPB + 16 * L.KTU) * (kTrsPB + 1)) * sizeof(T) + L.RW * sizeof(int);
     if (fwd_lds > 160 * 1024 || bwd_lds > 160 * 1024 || prep_lds > 160 * 1024) return 0;
     const size_t recs = (size_t)L.np * L.per_panel * sizeof(T);
     const size_t idxs = (size_t)L.np * L.idx_u16 * 2;
@@ -622,7 +635,7 @@ int trs_blocked_prepare(i64 n, i64 kl, i64 ku, const T *ab, i64 ldab, const i64 
     const size_t recs = (size_t)L.np * L.per_panel * sizeof(T);
     T *rec = (T *)work;
     unsigned short *idx = (unsigned short *)((char *)work + ((recs + 255) & ~(size_t)255));
-    const size_t lds = ((size_t)(L.RW + 2 * kTrsPB + 16 * L.KTU) * (kTrsPB + 1)) * sizeof(T) + 2 * L.RW * sizeof(int);
+    const size_t lds = ((size_t)(L.RW + 3 * kTrsPB + 16 * L.KTU) * (kTrsPB + 1)) * sizeof(T) + L.RW * sizeof(int);
     auto kern = trs_prep<T, kTrsPB>;
     if (lds > 64 * 1024)
         BH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -697,10 +710,10 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
                                CutSet{kd, (int)kl + 1, kd, 1}, 5, flags);
             hipLaunchKernelGGL(kf, dim3(grid.x, gl.p), block, fl, st, (const T *)B, ldb, Y, n, (int)nrhs, L, idx, rec,
                                SweepCut<T>{gl, flags, snl});
-            hipLaunchKernelGGL(sweep_check<T>, dim3(gl.p - 1, grid.x), dim3(64), 0, st, (const T *)snl, cl, flags);
+            hipLaunchKernelGGL(sweep_check<T>, dim3(gl.p - 1, grid.x), dim3(256), 0, st, (const T *)snl, cl, flags);
             hipLaunchKernelGGL(kb, dim3(grid.x, gu.p), block, bl, st, (const T *)Y, n, Z, n, (int)nrhs, L, rec, RB,
                                SweepCut<T>{gu, flags, snu});
-            hipLaunchKernelGGL(sweep_check<T>, dim3(gu.p - 1, grid.x), dim3(64), 0, st, (const T *)snu, cu, flags);
+            hipLaunchKernelGGL(sweep_check<T>, dim3(gu.p - 1, grid.x), dim3(256), 0, st, (const T *)snu, cu, flags);
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n,
                                (const T *)Z, B, 1, ldb, (const int *)flags);
             cut.flags = flags;
