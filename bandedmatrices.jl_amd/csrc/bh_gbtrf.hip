@@ -136,7 +136,8 @@ __global__ void __launch_bounds__(kLuThreads) gbtf2_single(LuSys<T> s, i64 *info
 template <typename T>
 int reg_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
 template <typename T>
-int blk_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
+int blk_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                     const LuCut<T> *cut);
 template <typename T>
 int small_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st);
 template <typename T>
@@ -251,14 +252,30 @@ static CutGeom lu_cut_geom(i64 n, i64 kl, i64 ku, i64 blocks, int tries) {
 // verdict in seq->flags, for the sequential kernel launched next (which does
 // nothing where the blocks succeeded) and to be freed after it; nullptr when
 // no blocks ran.
+int blk_shape_for(i64 kl, i64 ku);
+size_t mfma_lds_bytes(i64 kl, i64 elem);
+
+enum LuKernel { kLuNone, kLuMfma, kLuLane, kLuBlk };
+
 template <typename T>
-static int gbtrf_cut(bool mfma, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, void **ws_out, LuCut<T> *seq) {
+static int lu_kernel_launch(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo,
+                            hipStream_t st, const LuCut<T> *cut) {
+    switch (kind) {
+        case kLuMfma: return mfma_gbtrf_launch<T>(n, n, kl, ku, ab, ldab, ipiv, dinfo, st, cut);
+        case kLuLane: return lane_gbtrf_launch(n, n, kl, ku, ab, ldab, ipiv, dinfo, st, cut);
+        case kLuBlk: return blk_gbtrf_launch<T>(n, n, kl, ku, ab, ldab, ipiv, dinfo, st, cut);
+        default: return -1;
+    }
+}
+
+template <typename T>
+static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, void **ws_out, LuCut<T> *seq) {
     *ws_out = nullptr;
     if (kl < 1 || !cut_enabled()) return BH_OK;
     hipStream_t st = stream();
     const int kv = (int)(kl + ku), H = (int)(2 * kl + ku + 1);
-    // one workgroup per CU for the MFMA kernel (its LDS), one wave per SIMD for the lane kernel
-    const i64 blocks = mfma ? 256 : 1024;
+    // one workgroup per CU for the MFMA and the blocked kernel (their LDS), one wave per SIMD for the lane kernel
+    const i64 blocks = kind == kLuLane ? 1024 : 256;
     for (int tries = 0; tries < 2; ++tries) {
         const CutGeom g = lu_cut_geom<T>(n, kl, ku, blocks, tries);
         if (g.p == 0) return BH_OK;
@@ -272,8 +289,7 @@ static int gbtrf_cut(bool mfma, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipi
                            CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, flags);
         const unsigned gx = (unsigned)imin(64, cdiv((i64)g.span() * H, 1024));
         hipLaunchKernelGGL(lu_cut_copy<T>, dim3(gx, g.p), dim3(256), 0, st, cut, (const T *)ab, ldab, kv);
-        int r = mfma ? mfma_gbtrf_launch<T>(n, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut)
-                     : lane_gbtrf_launch(n, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);
+        const int r = lu_kernel_launch<T>(kind, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);
         if (r != BH_OK) {
             cut_free(ws, st);
             return r == -1 ? BH_OK : r;  // -1: the kernel does not take this band
@@ -324,11 +340,18 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
     const int ov = lu_kernel_override();
     int st = -1;
     const bool mfma = ov == 5 || (ov == 0 && ((ku >= 65 && kl >= 32) || (kl >= 8 && ku >= 8 && imin(m, n) >= kLongLu)));
-    const bool lane = !mfma && ov == 0 && (kl <= 8 || kl == 16) && kl + ku <= 63 && !getenv("BANDEDHIP_SMALL_LU");
+    LuKernel kind = kLuNone;  // the kernel that runs the system, where it has a form for blocks
+    const size_t ml = mfma_lds_bytes(kl, sizeof(T));
+    if (mfma)
+        kind = ml > 0 && ml + 4096 <= 160 * 1024 ? kLuMfma : kLuNone;
+    else if (ov == 0 && kl <= 16 && kl + ku <= 63 && !getenv("BANDEDHIP_SMALL_LU"))
+        kind = kLuLane;
+    else if (ov == 0 && kl >= 16 && blk_shape_for(kl, ku) >= 0)
+        kind = kLuBlk;
     void *ws = nullptr;
     LuCut<T> seq{};
-    if (m == n && (mfma || lane)) {
-        const int cs = gbtrf_cut<T>(mfma, n, kl, ku, ab, ldab, ipiv, &ws, &seq);
+    if (m == n && kind != kLuNone) {
+        const int cs = gbtrf_cut<T>(kind, n, kl, ku, ab, ldab, ipiv, &ws, &seq);
         if (cs) return cs;
     }
     struct Free {
@@ -345,7 +368,7 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
     if (mfma)
         st = mfma_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), ws ? &seq : nullptr);
     else if (ws)
-        st = lane_gbtrf_launch(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), &seq);
+        st = lu_kernel_launch<T>(kind, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), &seq);
     if (st == -1 && ws) {
         // the blocks' kernel does not take the whole system (its 32-bit
         // offsets): only their verdict tells whether another one has to run
@@ -354,12 +377,12 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
         BH_HIP(hipStreamSynchronize(stream()));
         if (fl[0] == 0 && fl[1] == 0) return BH_OK;
     }
-    // The one-wave lane kernel exists for kl <= 8 and kl = 16; above 16 the
+    // The one-wave lane kernel exists for kl <= 16; above 16 the
     // blocked kernel beats the generic one-wave kernel (at n = 65536, (24,24):
     // 113.5 ms against 278.6 ms, identical factors), so it goes first there.
     if (st == -1 && (ov == 4 || (ov == 0 && kl <= 16))) st = small_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream());
     if (st == -1 && (ov == 1 || (ov == 0 && kl >= 16)))
-        st = blk_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream());
+        st = blk_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), nullptr);
     if (st == -1 && ov != 3) st = reg_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream());
     if (st == -1) {
         LuSys<T> s{ab, ipiv, m, n, kl, ku, ldab};

@@ -35,6 +35,7 @@
 //      written to AB and the rows entering next prefetched early in it.
 // All barriers order LDS only.
 #include "bh_common.hpp"
+#include "bh_cut.hpp"
 
 namespace bh {
 
@@ -49,6 +50,7 @@ struct BlkArgs {
     i64 *info;
     int m, n, kl, ku;
     i64 ldab;
+    LuCut<T> cut;  // cut.g.p > 0: one workgroup per block of a cut system (bh_cut.hpp)
 };
 
 __device__ __forceinline__ int imin32(int a, int b) { return a < b ? a : b; }
@@ -131,6 +133,18 @@ __global__ void __launch_bounds__(64 * (NW + 1)) gbtrf_blk_kernel(BlkArgs<T> s) 
     using G = BlkGeom<T, NW, RRW, CCL>;
     constexpr int RS = G::RS, PR = G::PR, RSP = G::RSP, KVP = G::KVP, NWT = G::NWT, RRWP = G::RRWP;
     constexpr int NPRE = G::NPRE;
+    if (s.cut.g.p > 0) {  // this workgroup's block of a cut system
+        if (cut_closed(s.cut.flags)) return;
+        const int blk = blockIdx.x;
+        s.ab = s.cut.block_ab(blk);
+        s.ldab = s.cut.H;
+        s.m = s.cut.rows(blk);
+        s.n = s.cut.cols(blk);
+        s.ipiv = s.cut.ipiv + (i64)blk * s.cut.g.span();
+        s.info = s.cut.info + 2 * blk;
+    } else if (s.cut.flags && !cut_failed(s.cut.flags)) {
+        return;  // the blocks of a cut system have done it
+    }
     const int m = s.m, n = s.n, kl = s.kl, ku = s.ku, kv = kl + ku, H = kv + 1;
     const i64 ld = s.ldab;
     T *__restrict__ ab = s.ab;
@@ -606,7 +620,7 @@ int blk_launch_one(const BlkArgs<T> &a, hipStream_t st) {
     auto kern = gbtrf_blk_kernel<T, NW, RRW, CCL>;
     if (lds > 64 * 1024)
         BH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(1), dim3(64 * (NW + 1)), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.cut.g.p > 0 ? a.cut.g.p : 1), dim3(64 * (NW + 1)), lds, st, a);
     BH_LAUNCH_CHECK();
     return BH_OK;
 }
@@ -623,13 +637,14 @@ int blk_shape_for(i64 kl, i64 ku) {
 }
 
 template <typename T>
-int blk_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st) {
+int blk_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                     const LuCut<T> *cut) {
     if (blk_shape_for(kl, ku) < 0 || m >= (1ll << 30) || n >= (1ll << 30)) return -1;
-    BlkArgs<T> a{ab, ipiv, dinfo, (int)m, (int)n, (int)kl, (int)ku, ldab};
+    BlkArgs<T> a{ab, ipiv, dinfo, (int)m, (int)n, (int)kl, (int)ku, ldab, cut ? *cut : LuCut<T>{}};
     return blk_launch_one<T, 15, 10, 4>(a, st);
 }
 
-template int blk_gbtrf_launch<double>(i64, i64, i64, i64, double *, i64, i64 *, i64 *, hipStream_t);
-template int blk_gbtrf_launch<float>(i64, i64, i64, i64, float *, i64, i64 *, i64 *, hipStream_t);
+template int blk_gbtrf_launch<double>(i64, i64, i64, i64, double *, i64, i64 *, i64 *, hipStream_t, const LuCut<double> *);
+template int blk_gbtrf_launch<float>(i64, i64, i64, i64, float *, i64, i64 *, i64 *, hipStream_t, const LuCut<float> *);
 
 }  // namespace bh

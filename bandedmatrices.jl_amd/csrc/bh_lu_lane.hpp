@@ -29,14 +29,18 @@ struct BatchDesc {
     int n, kl, ku, cls, sys;
 };
 
-// Single-system gbtrf through the rotating-register kernel (kl <= 8 or
-// kl = 16, kl + ku <= 63, band storage under 2 GiB), or -1.  With a cut it
+// Single-system gbtrf through the rotating-register kernel (kl <= 16, kl + ku <= 63, band storage under 2 GiB), or -1.  With a cut it
 // runs the blocks of a cut system, one wave each; with cut->g.p == 0 it does
 // nothing unless cut->flags say that the blocks failed.
 int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, double *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<double> *cut);
 int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, float *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<float> *cut);
+// its widths 9 .. 15, compiled in units of their own (bh_lu_lane_wide_{d,s}.hip)
+int lane_gbtrf_launch_wide(i64 m, i64 n, i64 kl, i64 ku, double *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                           const LuCut<double> *cut);
+int lane_gbtrf_launch_wide(i64 m, i64 n, i64 kl, i64 ku, float *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                           const LuCut<float> *cut);
 // The persistent batched gbsv kernel over a schedule of nsys descriptors.
 int lane_batch_launch(unsigned blocks, unsigned threads, hipStream_t st, const BatchDesc *desc, int nsys, double *AB,
                       double *B, i64 *ipiv, i64 *info);
@@ -410,6 +414,34 @@ __global__ void __launch_bounds__(256) gbsv_batched_kernel(const BatchDesc *__re
 
 }  // namespace
 
+#ifdef BH_LANE_WIDE
+int lane_gbtrf_launch_wide(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
+                      const LuCut<BH_LANE_T> *cut) {
+    using T = BH_LANE_T;
+    const i64 nb = cut && cut->g.p > 0 ? cut->g.span() : n;  // a block's copy holds span() columns
+    if (kl + ku > 63 || m >= (1ll << 30) || n >= (1ll << 30) || ldab * nb * (i64)sizeof(T) >= (1ll << 31) ||
+        ldab * (i64)sizeof(T) >= (1ll << 24))
+        return -1;
+    const int mi = (int)m, ni = (int)n, ui = (int)ku;
+    const LuCut<T> c = cut ? *cut : LuCut<T>{};
+    const dim3 grid(c.g.p > 0 ? (unsigned)c.g.p : 1u);
+    switch ((int)kl) {
+#define BH_LANE_CASE(KLv)                                                                                       \
+    case KLv:                                                                                                   \
+        hipLaunchKernelGGL((gbtrf_lane_kernel<T, KLv>), grid, dim3(64), 0, st, mi, ni, ui, ab, ldab, ipiv,      \
+                           dinfo, c);                                                                           \
+        break;
+        BH_LANE_CASE(9) BH_LANE_CASE(10) BH_LANE_CASE(11) BH_LANE_CASE(12) BH_LANE_CASE(13) BH_LANE_CASE(14)
+        BH_LANE_CASE(15)
+#undef BH_LANE_CASE
+        default:
+            return -1;
+    }
+    BH_LAUNCH_CHECK();
+    return BH_OK;
+}
+
+#else
 int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<BH_LANE_T> *cut) {
     using T = BH_LANE_T;
@@ -430,7 +462,7 @@ int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, BH_LANE_T *ab, i64 ldab, i64
         BH_LANE_CASE(5) BH_LANE_CASE(6) BH_LANE_CASE(7) BH_LANE_CASE(8) BH_LANE_CASE(16)
 #undef BH_LANE_CASE
         default:
-            return -1;
+            return kl <= 15 ? lane_gbtrf_launch_wide(m, n, kl, ku, ab, ldab, ipiv, dinfo, st, cut) : -1;
     }
     BH_LAUNCH_CHECK();
     return BH_OK;
@@ -443,6 +475,7 @@ int lane_batch_launch(unsigned blocks, unsigned threads, hipStream_t st, const B
     BH_LAUNCH_CHECK();
     return BH_OK;
 }
+#endif  // BH_LANE_WIDE
 #endif  // BH_LANE_T
 
 }  // namespace bh

@@ -266,7 +266,7 @@ int small_class(i64 kl) {
 }  // namespace
 
 // Single-system narrow-band LU (kl + ku <= 63, kl <= 31), or -1.  The
-// rotating-register kernel runs for kl <= 8 and kl = 16 when the band
+// rotating-register kernel runs for kl <= 16 when the band
 // storage is under 2 GiB (its buffer offsets are 32-bit); other widths, and
 // BANDEDHIP_SMALL_LU=class, take the register-class kernel.
 template <typename T>

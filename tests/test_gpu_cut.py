@@ -50,6 +50,8 @@ def _system(rng, n, kl, ku, dtype, kind):
 LU = [  # n, kl, ku: lane kernel, its edges; the MFMA kernel for long and for wide bands
     (1000, 1, 1), (1003, 2, 5), (4096, 4, 4), (10000, 4, 3), (10001, 8, 8), (5000, 16, 3), (16383, 8, 8),
     (16384, 8, 8), (16400, 16, 16), (262144, 9, 9), (30001, 9, 20), (9000, 64, 70), (12345, 100, 128), (3000, 33, 65),
+    (5000, 9, 2), (6001, 11, 5), (20000, 13, 3), (7000, 15, 16),  # the lane kernel's wider half
+    (5000, 20, 20), (12000, 40, 50), (6000, 16, 50), (9000, 70, 60),  # the blocked kernel
 ]
 
 
