@@ -162,8 +162,8 @@ __global__ void __launch_bounds__(64) gbqrf_lane(int m, int n, int u, T *D, i64 
         // outputs: row k of the window's columns, the reflector from lanes 1 .. L
         const int rowb = k * ldb + ub;
         ql_st(rD, d <= last ? (int)__umul24(d, dstep) : -1, rowb, r0);
-        // (unscaled when the column is zero: it stands as it is)
-        ql_st(rD, some && lane >= 1 && lane < len ? lane * SZ : -1, rowb, quo);
+        // (a column whose squares sum to zero stands as the updates left it)
+        ql_st(rD, lane >= 1 && lane < len ? lane * SZ : -1, rowb, some ? quo : num);
 #pragma unroll
         for (int i = 1; i < R; ++i)
             if (!TAIL || i < len) {

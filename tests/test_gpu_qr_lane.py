@@ -46,3 +46,21 @@ def test_single_precision(bh, m, n, l, u):
     if m < n:  # the last row's reflector is the identity: R holds what the band stores of it
         got = np.triu(got)
     assert np.abs(got - R).max() <= 60 * np.finfo(np.float32).eps * np.abs(R).max()
+
+
+@pytest.mark.parametrize("l,u", [(1, 1), (4, 4), (7, 3)])
+@pytest.mark.parametrize("low,high", [(-90, -89), (89, 91), (-160, -150), (150, 153), (-120, 120), (-300, -290)])
+def test_exponents(bh, oracle, l, u, low, high):
+    """Entries whose squares overflow or vanish: a column whose squares sum to zero keeps what the earlier
+    reflectors made of it."""
+    m = n = 300
+    rng = np.random.default_rng(l + 100 * (high + 400))
+    A = band(rng, l, u, n, np.float64, dist="n") * 10.0 ** rng.uniform(low, high, (l + u + 1, n))
+    A[:, 40] = 0
+    A[u, 80] = 0
+    with np.errstate(all="ignore"):
+        D, tau = oracle.gbqrf(m, n, l, l + u, oracle.pad_for_lu(np.asfortranarray(A), m, n, l, u))
+    F = bh.qr(bh.BandedMatrix.from_host(np.asfortranarray(A), m, l, u))
+    got, nan = F.factors.host_data(), np.isnan(D)
+    assert (np.isnan(got) == nan).all() and bits_equal(np.where(nan, 0, got), np.where(nan, 0, D))
+    assert np.array_equal(F.tau.numpy()[:n], tau, equal_nan=True)
