@@ -181,11 +181,21 @@ struct CutBuf {
     bool busy = false;
     unsigned long long used = 0;
 };
+// Allocations, frees and waits of a call on one stream are legal while another
+// stream is captured in the global mode only from a thread whose own mode is
+// relaxed; otherwise they fail and spoil that capture.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 struct CutBufs {
     CutBuf b[4];
     unsigned long long clock = 0;
     int off = 0;
     ~CutBufs() {
+        const RelaxedCapture relaxed;
         for (CutBuf &c : b) {
             if (c.p) (void)hipFree(c.p);
             if (c.done) (void)hipEventDestroy(c.done);
@@ -222,6 +232,7 @@ void *cut_alloc(size_t bytes, hipStream_t st) {
         if (!c || x.used < c->used) c = &x;
     }
     if (!c) return nullptr;
+    const RelaxedCapture relaxed;
     bool ok = true;
     if (c->p && (c->dev != dev || c->bytes < bytes)) {
         ok = hipEventSynchronize(c->done) == hipSuccess && hipFree(c->p) == hipSuccess;
@@ -257,6 +268,7 @@ void cut_free(void *p, hipStream_t st) {
     for (CutBuf &c : g_cut.b) {
         if (c.p != p) continue;
         if (c.bytes > kCutKeep || hipEventRecord(c.done, st) != hipSuccess) {
+            const RelaxedCapture relaxed;
             (void)hipStreamSynchronize(st);
             (void)hipFree(c.p);
             c.p = nullptr;

@@ -5,6 +5,7 @@ lead-in's rounding is checked, not trusted.  Inputs that must fall back (weak
 diagonals, a zero column, a NaN, interchanges) are mixed with dominant ones,
 at sizes around the edges of the blocks."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -259,3 +260,38 @@ def test_cholesky_narrow(bh, monkeypatch, dtype, kd):
         on, off = _both(monkeypatch, run)
         assert off[1] == 0
         _same(on, off)
+
+
+def test_other_stream_captured(bh, monkeypatch):
+    """A call that waits for nothing, of a new thread, whose buffers are allocated by it, while another stream is
+    captured: that stays valid.  (Calls that read a result back, like pbtrf, are refused then, cut or not.)"""
+    hip = C.CDLL(bh._lib.LIB_PATH)  # the runtime's own symbols, through the library's dependency on it
+    n, k = 300007, 3
+    ab = np.ones((k + 1, n), order="F")
+    ab[k] = 9
+    A, b = bh.DeviceArray.from_numpy(ab), np.random.default_rng(3).standard_normal(n)
+
+    def solve(x, errors):
+        try:
+            bh._lib.call("bh_dtbsv", b"U", b"N", b"N", n, k, A.ptr, k + 1, x.ptr, 1)
+        except Exception as e:
+            errors.append(e)
+
+    def run():
+        x, errors = bh.DeviceArray.from_numpy(b), []
+        a, g = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamCreate(C.byref(a)) == 0
+        assert hip.hipStreamBeginCapture(a, C.c_int(0)) == 0
+        t = threading.Thread(target=solve, args=(x, errors))
+        t.start()
+        t.join()
+        assert hip.hipStreamEndCapture(a, C.byref(g)) == 0
+        if g.value:
+            assert hip.hipGraphDestroy(g) == 0
+        assert hip.hipStreamDestroy(a) == 0
+        assert not errors
+        return (x.numpy(),)
+
+    x = bh.DeviceArray.from_numpy(b)
+    solve(x, [])  # the kernels loaded before the capture
+    _same(*_both(monkeypatch, run))
