@@ -12,7 +12,7 @@ from __future__ import annotations
 import ctypes as C
 
 from . import _lib
-from .bandedmatrix import BandedMatrix, _prefix, mul
+from .bandedmatrix import BandedMatrix, DimensionMismatch, _prefix, mul
 from .device import DeviceArray
 from .lu import BandedLU, ldiv_, lu
 
@@ -55,6 +55,12 @@ def loss_and_grad(A: BandedMatrix, b: DeviceArray, w: DeviceArray, x0: DeviceArr
     factors and pivots, then one fused band kernel
     dA_ij = fma(y0_i, x0_j, -(lambda_i x_j))."""
     n = A.shape[0]
+    # L is a number: one right-hand side (a single column counts) and one weight
+    # vector; the kernels below take bare pointers and would read column 0 of more
+    if b.shape not in ((n,), (n, 1)):
+        raise DimensionMismatch(f"b must be one vector of length {n}, has shape {b.shape}")
+    if w.shape != (n,) and not (n == 1 and w.shape == (1, 1)):
+        raise DimensionMismatch(f"w must be a vector of length {n}, has shape {w.shape}")
     F = lu(A)
     x = ldiv_(F, b.copy(), method)
     y0 = DeviceArray((n,), A.dtype)
