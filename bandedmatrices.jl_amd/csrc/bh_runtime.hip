@@ -5,10 +5,7 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <mutex>
-#include <unordered_map>
-#include <vector>
-
+#include "bh_blocks.hpp"
 #include "bh_common.hpp"
 #include "bh_cut.hpp"
 
@@ -76,96 +73,20 @@ int scratch_buffer(size_t bytes, void **p) {
     return BH_OK;
 }
 
-// ---- large blocks of bh_malloc.  Mapping and unmapping one costs far more
-// than the work of many calls (hipMalloc + hipFree: 4 us at 2 MB, 28 at 16 MB,
-// 280 at 69-103 MB), and a program that factors in a loop frees what it is
-// about to ask for.  So bh_free keeps blocks of at least kBlockMin, up to kBlockKeep
-// bytes in all, after waiting for the device as hipFree does (no work of any
-// stream can still touch a kept block); the oldest go back when there is no
-// room, those not asked for over kBlockAge frees, and all of them when the device runs out.
-constexpr size_t kBlockMin = size_t(8) << 20;
-constexpr size_t kBlockKeep = size_t(1) << 30;
-constexpr unsigned long long kBlockAge = 64;
-struct Block {
-    void *p;
-    size_t bytes;
-    int dev;
-    unsigned long long at;
-};
-static std::mutex g_block_mutex;
-static std::unordered_map<void *, Block> *g_blocks = new std::unordered_map<void *, Block>;  // in use
-static std::vector<Block> *g_kept = new std::vector<Block>;                                  // oldest first
-static size_t g_kept_bytes = 0;
-static unsigned long long g_block_clock = 0;
-
-// Give back the kept blocks past `age` frees, then the oldest until `bytes`
-// more fit.  The mutex is held.
-static void blocks_trim(unsigned long long age, size_t bytes) {
-    auto &k = *g_kept;
-    size_t i = 0;
-    while (i < k.size() && (g_block_clock - k[i].at > age || g_kept_bytes + bytes > kBlockKeep)) {
-        (void)hipFree(k[i].p);
-        g_kept_bytes -= k[i].bytes;
-        ++i;
-    }
-    k.erase(k.begin(), k.begin() + i);
-}
-
-static hipError_t block_malloc(void **p, size_t bytes) {
-    int dev = -1;
-    if (bytes < kBlockMin || hipGetDevice(&dev) != hipSuccess) return hipMalloc(p, bytes);
-    std::lock_guard<std::mutex> lock(g_block_mutex);
-    auto &k = *g_kept;
-    size_t best = k.size();
-    for (size_t i = 0; i < k.size(); ++i)
-        if (k[i].dev == dev && k[i].bytes >= bytes && k[i].bytes <= bytes + bytes / 8 &&
-            (best == k.size() || k[i].bytes < k[best].bytes))
-            best = i;
-    if (best < k.size()) {
-        *p = k[best].p;
-        g_kept_bytes -= k[best].bytes;
-        (*g_blocks)[*p] = k[best];
-        k.erase(k.begin() + best);
-        return hipSuccess;
-    }
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory && !k.empty()) {
-        (void)hipGetLastError();
-        blocks_trim(0, kBlockKeep);
-        e = hipMalloc(p, bytes);
-    }
-    if (e == hipSuccess) (*g_blocks)[*p] = Block{*p, bytes, dev, 0};
-    return e;
-}
-
-static hipError_t block_free(void *p) {
-    int dev = -1;
-    std::unique_lock<std::mutex> lock(g_block_mutex);
-    const auto it = g_blocks->find(p);
-    if (it == g_blocks->end()) {
-        lock.unlock();
-        return hipFree(p);
-    }
-    Block b = it->second;
-    g_blocks->erase(it);
-    ++g_block_clock;
-    if (b.bytes > kBlockKeep / 2 || hipGetDevice(&dev) != hipSuccess || dev != b.dev) {
-        lock.unlock();
-        return hipFree(p);
-    }
-    lock.unlock();
-    const hipError_t e = hipDeviceSynchronize();  // what hipFree waits for
-    if (e != hipSuccess) {
-        (void)hipFree(p);
+// ---- large blocks of bh_malloc (bh_blocks.hpp)
+struct HipDevice {
+    static constexpr int kNoMemory = hipErrorOutOfMemory, kBadPointer = hipErrorInvalidValue;
+    int current(int *dev) { return hipGetDevice(dev); }
+    int alloc(void **p, size_t bytes) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e == hipErrorOutOfMemory) (void)hipGetLastError();
         return e;
     }
-    lock.lock();
-    blocks_trim(kBlockAge, b.bytes);
-    b.at = g_block_clock;
-    g_kept->push_back(b);
-    g_kept_bytes += b.bytes;
-    return hipSuccess;
-}
+    int release(void *p) { return hipFree(p); }
+    int wait() { return hipDeviceSynchronize(); }
+};
+// never destroyed: arrays may be freed while the process ends
+static BlockCache<HipDevice> &g_blocks = *new BlockCache<HipDevice>;
 
 // ---- memory of the cut paths (bh_cut.hpp).  Each thread keeps up to four
 // buffers of at most kCutKeep bytes, one to a stream, and frees them when it ends;
@@ -336,13 +257,13 @@ int bh_malloc(void **dptr, size_t bytes) {
     if (st) return st;
     *dptr = nullptr;
     if (bytes == 0) return BH_OK;
-    BH_HIP(block_malloc(dptr, bytes));
+    BH_HIP((hipError_t)g_blocks.take(dptr, bytes));
     return BH_OK;
 }
 
 int bh_free(void *dptr) {
     if (dptr == nullptr) return BH_OK;
-    BH_HIP(block_free(dptr));
+    BH_HIP((hipError_t)g_blocks.give(dptr));
     return BH_OK;
 }
 
