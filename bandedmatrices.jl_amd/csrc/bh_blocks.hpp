@@ -80,12 +80,11 @@ class BlockCache {
         lock.unlock();
         const int e = dev_.wait();  // what a free waits for
         lock.lock();
-        used_.erase(p);
-        if (e != 0) {
-            lock.unlock();
-            (void)dev_.release(p);
+        if (e != 0) {  // nothing is freed: the caller may try again
+            used_[p].leaving = false;
             return e;
         }
+        used_.erase(p);
         trim(kAge, b.bytes);
         b.at = clock_;
         b.leaving = false;

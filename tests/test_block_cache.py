@@ -70,6 +70,17 @@ int main() {  // never more than kKeep kept, the oldest go first, and unused one
     CHECK(c.kept_bytes() == 10 * M && S.live.size() == 1 && S.bad == 0);
     return 0;
 }""",
+    "wait_fails": r"""
+int main() {  // a free whose wait fails has freed nothing: the block is in use still, and a second try frees it
+    Cache c; void *p, *q;
+    CHECK(c.take(&p, 16 * M) == 0);
+    S.fail_wait = 7;
+    CHECK(c.give(p) == 7 && S.live.count(p) == 1 && c.kept_bytes() == 0);
+    CHECK(c.take(&q, 16 * M) == 0 && q != p);
+    S.fail_wait = 0;
+    CHECK(c.give(p) == 0 && c.give(p) == Dev::kBadPointer && c.give(q) == 0 && S.bad == 0 && c.kept_bytes() == 32 * M);
+    return 0;
+}""",
 }
 
 
