@@ -6,7 +6,7 @@ operator interface for the path: BandedMatrix storage, mul!/A*x, A*B, lu,
 ldiv!/\\, qr and the triangular band solve/product.
 """
 from ._lib import BandedHIPError, load as load_library, LIB_PATH
-from .device import DeviceArray, Timer, sync
+from .device import DeviceArray, Timer, sync, trim
 from .bandedmatrix import (BandedMatrix, BandError, DimensionMismatch, _BandedMatrix, axpy_, brand, convert, copyto_,
                            gbmm, mul, prodbandwidths)
 from .lu import BandedLU, SingularException, TransposeFact, ldiv_, lu, lu_, pad_for_lu, solve
@@ -20,7 +20,7 @@ from .tribanded import (BandView, LowerTriangular, UnitLowerTriangular, UnitUppe
                         tbsv_)
 
 __all__ = [
-    "BandedHIPError", "load_library", "LIB_PATH", "DeviceArray", "Timer", "sync", "BandedMatrix", "BandError",
+    "BandedHIPError", "load_library", "LIB_PATH", "DeviceArray", "Timer", "sync", "trim", "BandedMatrix", "BandError",
     "DimensionMismatch", "_BandedMatrix", "brand", "gbmm", "mul", "prodbandwidths", "BandedLU",
     "SingularException", "TransposeFact", "ldiv_", "lu", "lu_", "pad_for_lu", "solve", "MixedResult",
     "MixedSolver", "solve_mixed", "BandedQR", "QRPackedQ", "qr", "qr_", "qr_ldiv_", "qr_lmul_", "qr_rmul_", "qr_solve",

@@ -25,6 +25,7 @@ SIGNATURES: dict[str, tuple] = {
     "bh_last_error": (C.c_char_p, []),
     "bh_malloc": (C.c_int, [C.POINTER(vp), C.c_size_t]),
     "bh_free": (C.c_int, [vp]),
+    "bh_trim": (C.c_int, []),
     "bh_memcpy_htod": (C.c_int, [vp, vp, C.c_size_t]),
     "bh_memcpy_dtoh": (C.c_int, [vp, vp, C.c_size_t]),
     "bh_memcpy_dtod": (C.c_int, [vp, vp, C.c_size_t]),

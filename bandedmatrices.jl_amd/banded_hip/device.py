@@ -128,6 +128,13 @@ def sync() -> None:
     _lib.call("bh_sync")
 
 
+def trim() -> None:
+    """Give back the device memory the library keeps for later calls (freed
+    arrays of 8 MiB and more, and the buffers of the block paths), for other
+    allocators of the process."""
+    _lib.call("bh_trim")
+
+
 class Timer:
     """HIP events on the library stream; elapsed() synchronises the stop event."""
 

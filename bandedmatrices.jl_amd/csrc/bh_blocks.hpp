@@ -5,13 +5,14 @@
 // program that factors in a loop frees what it is about to ask for.  So a
 // freed block of at least kMin bytes is kept, up to kKeep bytes in all, after
 // waiting for the device as hipFree does (no work of any stream can still
-// touch a kept block); the oldest go back when there is no room, and those not
-// asked for over kAge frees.
+// touch a kept block); the oldest go back when there is no room, those not
+// asked for over kAge frees, and all of them when the device runs out.
 //
 // The bookkeeping only, without HIP's headers: Dev supplies the runtime (its
 // calls return 0 or an error code), so that it can be tested on the host.
 //   int current(int *dev)            the calling thread's device
 //   int alloc(void **p, size_t n), release(void *p), wait()
+//   void others()                    gives back what else is kept (the device ran out)
 //   static constexpr int kNoMemory, kBadPointer
 #pragma once
 #include <stddef.h>
@@ -33,8 +34,16 @@ class BlockCache {
 
     int take(void **p, size_t bytes) {
         int d = -1;
-        if (bytes < kMin || dev_.current(&d) != 0) return dev_.alloc(p, bytes);
-        std::lock_guard<std::mutex> lock(m_);
+        std::unique_lock<std::mutex> lock(m_, std::defer_lock);
+        const bool track = bytes >= kMin && dev_.current(&d) == 0;
+        if (!track) {
+            int e = dev_.alloc(p, bytes);
+            if (e != Dev::kNoMemory) return e;
+            drop();
+            dev_.others();
+            return dev_.alloc(p, bytes);
+        }
+        lock.lock();
         size_t best = kept_.size();
         for (size_t i = 0; i < kept_.size(); ++i)
             if (kept_[i].dev == d && kept_[i].bytes >= bytes && kept_[i].bytes <= bytes + bytes / 8 &&
@@ -48,8 +57,9 @@ class BlockCache {
             return 0;
         }
         int e = dev_.alloc(p, bytes);
-        if (e == Dev::kNoMemory && !kept_.empty()) {
+        if (e == Dev::kNoMemory) {
             trim(0, kKeep);
+            dev_.others();
             e = dev_.alloc(p, bytes);
         }
         if (e == 0) used_[*p] = Block{*p, bytes, d, 0, false};
@@ -91,6 +101,12 @@ class BlockCache {
         kept_.push_back(b);
         kept_bytes_ += b.bytes;
         return 0;
+    }
+
+    // Give back every kept block.
+    void drop() {
+        std::lock_guard<std::mutex> lock(m_);
+        trim(0, kKeep);
     }
 
     size_t kept_bytes() {

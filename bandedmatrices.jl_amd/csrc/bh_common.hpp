@@ -25,6 +25,10 @@ hipStream_t stream();
 // the library stream).
 int ctrl_words(i64 **p);
 int scratch_buffer(size_t bytes, void **p);
+// hipMalloc for the library's own use: when the device has none left, all that
+// is kept for later calls (freed blocks, idle buffers of the block paths) goes
+// back and it tries once more.
+hipError_t device_alloc(void **p, size_t bytes);
 // Looks up, with `device` current, the device address of the statically
 // allocated scratch used by bh_dsgbsv_noalloc (once per device).
 int noalloc_setup(int device);

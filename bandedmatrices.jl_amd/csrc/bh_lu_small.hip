@@ -370,7 +370,7 @@ int plan_set_order(bh_batch_plan *p, int kind) {
         (void)hipFree(p->desc);
         p->desc = nullptr;
         p->desc_cap = 0;
-        if (hipMalloc((void **)&p->desc, sizeof(BatchDesc) * len) != hipSuccess) {
+        if (device_alloc((void **)&p->desc, sizeof(BatchDesc) * len) != hipSuccess) {
             set_error("bh_batch plan: out of device memory");
             return BH_ERR_ALLOC;
         }
@@ -414,10 +414,10 @@ int batch_autotune(bh_batch_plan *p, const T *AB, const T *B, double *best_ms) {
         (void)hipFree(ip2);
         (void)hipFree(inf2);
     };
-    if (hipMalloc((void **)&ab2, sizeof(T) * p->ab_elems) != hipSuccess ||
-        hipMalloc((void **)&b2, sizeof(T) * p->vec_elems) != hipSuccess ||
-        hipMalloc((void **)&ip2, sizeof(i64) * p->vec_elems) != hipSuccess ||
-        hipMalloc((void **)&inf2, sizeof(i64) * p->nsys) != hipSuccess) {
+    if (device_alloc((void **)&ab2, sizeof(T) * p->ab_elems) != hipSuccess ||
+        device_alloc((void **)&b2, sizeof(T) * p->vec_elems) != hipSuccess ||
+        device_alloc((void **)&ip2, sizeof(i64) * p->vec_elems) != hipSuccess ||
+        device_alloc((void **)&inf2, sizeof(i64) * p->nsys) != hipSuccess) {
         cleanup();
         set_error("bh_batch_autotune: out of device memory");
         return BH_ERR_ALLOC;

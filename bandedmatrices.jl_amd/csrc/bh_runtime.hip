@@ -5,6 +5,10 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
 #include "bh_blocks.hpp"
 #include "bh_common.hpp"
 #include "bh_cut.hpp"
@@ -66,11 +70,86 @@ int scratch_buffer(size_t bytes, void **p) {
         g_scratch = nullptr;
         g_scratch_bytes = 0;
         const size_t nb = bytes + bytes / 2;
-        BH_HIP(hipMalloc(&g_scratch, nb));
+        BH_HIP(device_alloc(&g_scratch, nb));
         g_scratch_bytes = nb;
     }
     *p = g_scratch;
     return BH_OK;
+}
+
+// ---- memory of the cut paths (bh_cut.hpp).  Each thread keeps up to four
+// buffers of at most kCutKeep bytes, one to a stream, and frees them when it ends;
+// a fifth stream takes over the buffer unused for longest, behind its last
+// use.  (A stream-ordered pool of HIP's, tried first, cost 60-140 us a call
+// with a synchronisation between calls; this costs under 5.)
+struct CutBuf {
+    int dev = -1;
+    hipStream_t st = nullptr;
+    void *p = nullptr;
+    size_t bytes = 0;
+    hipEvent_t done = nullptr;  // behind the last call that used it
+    bool busy = false;          // a call of its thread has it: nobody else touches it
+    unsigned long long used = 0;
+};
+// Allocations, frees and waits of a call on one stream are legal while another
+// stream is captured in the global mode only from a thread whose own mode is
+// relaxed; otherwise they fail and spoil that capture.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Frees a buffer behind the work that used it; false: it could not be waited for.
+static bool cut_release(CutBuf &c) {
+    if (!c.p) return true;
+    if (hipEventSynchronize(c.done) != hipSuccess || hipFree(c.p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    c.p = nullptr;
+    c.bytes = 0;
+    return true;
+}
+
+struct CutBufs;
+// every thread's, so that memory can be had back from all of them (never
+// destroyed: threads may end after this unit's statics)
+static std::mutex &g_cut_mutex = *new std::mutex;
+static std::vector<CutBufs *> &g_cut_all = *new std::vector<CutBufs *>;
+
+struct CutBufs {
+    std::mutex m;  // the buffers' fields, but for those of a busy one
+    CutBuf b[4];
+    unsigned long long clock = 0;
+    int off = 0;
+    CutBufs() {
+        std::lock_guard<std::mutex> all(g_cut_mutex);
+        g_cut_all.push_back(this);
+    }
+    ~CutBufs() {
+        {
+            std::lock_guard<std::mutex> all(g_cut_mutex);
+            g_cut_all.erase(std::find(g_cut_all.begin(), g_cut_all.end(), this));
+        }
+        const RelaxedCapture relaxed;
+        for (CutBuf &c : b) {
+            if (c.p) (void)hipFree(c.p);
+            if (c.done) (void)hipEventDestroy(c.done);
+        }
+    }
+};
+static thread_local CutBufs g_cut;
+
+// The idle buffers of every thread.
+static void cut_release_idle() {
+    const RelaxedCapture relaxed;
+    std::lock_guard<std::mutex> all(g_cut_mutex);
+    for (CutBufs *t : g_cut_all) {
+        std::lock_guard<std::mutex> lock(t->m);
+        for (CutBuf &c : t->b)
+            if (!c.busy) (void)cut_release(c);
+    }
 }
 
 // ---- large blocks of bh_malloc (bh_blocks.hpp)
@@ -84,46 +163,23 @@ struct HipDevice {
     }
     int release(void *p) { return hipFree(p); }
     int wait() { return hipDeviceSynchronize(); }
+    void others() { cut_release_idle(); }
 };
 // never destroyed: arrays may be freed while the process ends
 static BlockCache<HipDevice> &g_blocks = *new BlockCache<HipDevice>;
 
-// ---- memory of the cut paths (bh_cut.hpp).  Each thread keeps up to four
-// buffers of at most kCutKeep bytes, one to a stream, and frees them when it ends;
-// a fifth stream takes over the buffer unused for longest, behind its last
-// use.  (A stream-ordered pool of HIP's, tried first, cost 60-140 us a call
-// with a synchronisation between calls; this costs under 5.)
-struct CutBuf {
-    int dev = -1;
-    hipStream_t st = nullptr;
-    void *p = nullptr;
-    size_t bytes = 0;
-    hipEvent_t done = nullptr;  // behind the last call that used it
-    bool busy = false;
-    unsigned long long used = 0;
-};
-// Allocations, frees and waits of a call on one stream are legal while another
-// stream is captured in the global mode only from a thread whose own mode is
-// relaxed; otherwise they fail and spoil that capture.
-struct RelaxedCapture {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-};
+static void release_kept() {
+    g_blocks.drop();
+    cut_release_idle();
+}
 
-struct CutBufs {
-    CutBuf b[4];
-    unsigned long long clock = 0;
-    int off = 0;
-    ~CutBufs() {
-        const RelaxedCapture relaxed;
-        for (CutBuf &c : b) {
-            if (c.p) (void)hipFree(c.p);
-            if (c.done) (void)hipEventDestroy(c.done);
-        }
-    }
-};
-static thread_local CutBufs g_cut;
+hipError_t device_alloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    release_kept();
+    return hipMalloc(p, bytes);
+}
 
 CutOff::CutOff() { ++g_cut.off; }
 CutOff::~CutOff() { --g_cut.off; }
@@ -144,55 +200,60 @@ void *cut_alloc(size_t bytes, hipStream_t st) {
     }
     if (cap != hipStreamCaptureStatusNone) return nullptr;
     CutBuf *c = nullptr;
-    for (CutBuf &x : g_cut.b) {
-        if (x.busy) continue;
-        if (x.p && x.dev == dev && x.st == st) {
-            c = &x;
-            break;
+    {
+        std::lock_guard<std::mutex> lock(g_cut.m);
+        for (CutBuf &x : g_cut.b) {
+            if (x.busy) continue;
+            if (x.p && x.dev == dev && x.st == st) {
+                c = &x;
+                break;
+            }
+            if (!c || x.used < c->used) c = &x;
         }
-        if (!c || x.used < c->used) c = &x;
+        if (!c) return nullptr;
+        c->busy = true;
     }
-    if (!c) return nullptr;
     const RelaxedCapture relaxed;
     bool ok = true;
-    if (c->p && (c->dev != dev || c->bytes < bytes)) {
-        ok = hipEventSynchronize(c->done) == hipSuccess && hipFree(c->p) == hipSuccess;
-        c->p = nullptr;
-        if (c->dev != dev) {
-            (void)hipEventDestroy(c->done);
-            c->done = nullptr;
-        }
-    } else if (c->p && c->st != st) {
+    if (c->p && (c->dev != dev || c->bytes < bytes))
+        ok = cut_release(*c);
+    else if (c->p && c->st != st)
         ok = hipStreamWaitEvent(st, c->done, 0) == hipSuccess;
+    if (ok && c->done && c->dev != dev) {
+        (void)hipEventDestroy(c->done);
+        c->done = nullptr;
     }
     if (ok && !c->done) ok = hipEventCreateWithFlags(&c->done, hipEventDisableTiming) == hipSuccess;
     if (ok && !c->p) {
         // some room to grow, within what is kept
         const size_t nb = bytes > kCutKeep ? bytes : (bytes + bytes / 4 < kCutKeep ? bytes + bytes / 4 : kCutKeep);
-        ok = hipMalloc(&c->p, nb) == hipSuccess;
+        ok = device_alloc(&c->p, nb) == hipSuccess;
         c->bytes = ok ? nb : 0;
         if (!ok) c->p = nullptr;
     }
     if (!ok) {
         (void)hipGetLastError();
+        std::lock_guard<std::mutex> lock(g_cut.m);
+        c->busy = false;
         return nullptr;
     }
     c->dev = dev;
     c->st = st;
-    c->busy = true;
     c->used = ++g_cut.clock;
     return c->p;
 }
 
 void cut_free(void *p, hipStream_t st) {
     if (!p) return;
+    std::lock_guard<std::mutex> lock(g_cut.m);
     for (CutBuf &c : g_cut.b) {
-        if (c.p != p) continue;
+        if (!c.busy || c.p != p) continue;
         if (c.bytes > kCutKeep || hipEventRecord(c.done, st) != hipSuccess) {
             const RelaxedCapture relaxed;
             (void)hipStreamSynchronize(st);
             (void)hipFree(c.p);
             c.p = nullptr;
+            c.bytes = 0;
             (void)hipGetLastError();
         }
         c.busy = false;
@@ -264,6 +325,11 @@ int bh_malloc(void **dptr, size_t bytes) {
 int bh_free(void *dptr) {
     if (dptr == nullptr) return BH_OK;
     BH_HIP((hipError_t)g_blocks.give(dptr));
+    return BH_OK;
+}
+
+int bh_trim(void) {
+    release_kept();
     return BH_OK;
 }
 

@@ -48,6 +48,12 @@ int bh_device_count(int *count);
 const char *bh_last_error(void);
 int bh_malloc(void **dptr, size_t bytes);
 int bh_free(void *dptr);
+/* Gives back the device memory the library keeps for later calls: blocks that
+ * bh_free keeps for bh_malloc (up to 1 GiB) and the buffers that calls run by
+ * blocks keep per thread (up to four of 2 GiB), those of every thread that no
+ * call uses just then.  Waits for the work that used them.  It happens by
+ * itself when an allocation of the library finds none left. */
+int bh_trim(void);
 int bh_memcpy_htod(void *dst, const void *src_host, size_t bytes);
 int bh_memcpy_dtoh(void *dst_host, const void *src, size_t bytes);
 int bh_memcpy_dtod(void *dst, const void *src, size_t bytes);

@@ -18,6 +18,7 @@ HOST = r"""
 // Addresses are numbers: alloc hands out new ones, release of one that is not
 // live is what a runtime reports (and what must never be asked for a kept block).
 struct State { std::set<void*> live; size_t next = 4096, limit = ~size_t(0), bytes = 0; int released = 0, bad = 0, fail_wait = 0;
+               size_t elsewhere = 0;
                std::set<size_t> sizes; size_t size_of[4096]; };
 static State S;
 struct Dev {
@@ -32,6 +33,7 @@ struct Dev {
         S.bytes -= S.size_of[(size_t)p / 4096]; ++S.released; return 0;
     }
     int wait() { return S.fail_wait; }
+    void others() { S.bytes -= S.elsewhere; S.elsewhere = 0; }
 };
 #define CHECK(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
 typedef bh::BlockCache<Dev> Cache;
@@ -81,6 +83,25 @@ int main() {  // a free whose wait fails has freed nothing: the block is in use 
     CHECK(c.give(p) == 0 && c.give(p) == Dev::kBadPointer && c.give(q) == 0 && S.bad == 0 && c.kept_bytes() == 32 * M);
     return 0;
 }""",
+    "out_of_memory": r"""
+int main() {  // a request of any size has the kept blocks, and what is kept elsewhere, given back before it fails
+    for (size_t want : {size_t(4096), M, 16 * M, 64 * M}) {
+        Cache c; void *p, *q;
+        S = State(); S.limit = 100 * M;
+        CHECK(c.take(&p, 48 * M) == 0 && c.take(&q, 48 * M) == 0 && c.give(p) == 0 && c.give(q) == 0);
+        S.limit = 96 * M;
+        CHECK(c.take(&p, want) == 0 && c.kept_bytes() == 0 && S.bytes == want);
+        S.elsewhere = S.limit - S.bytes; S.bytes = S.limit;
+        CHECK(c.take(&q, want / 4) == 0 && S.elsewhere == 0);
+        CHECK(c.take(&q, 97 * M) == Dev::kNoMemory && S.bad == 0);
+    }
+    Cache c; void *p;
+    S = State();
+    CHECK(c.take(&p, 48 * M) == 0 && c.give(p) == 0);
+    c.drop();
+    CHECK(c.kept_bytes() == 0 && S.live.empty() && c.give(p) == Dev::kBadPointer);
+    return 0;
+}""",
 }
 
 
@@ -113,3 +134,52 @@ def test_freed_twice(bh):
     for v, h in ((q, a), (r, b)):
         assert L.bh_memcpy_dtoh(got.ctypes.data, v, n) == 0 and np.array_equal(got, h)
     assert L.bh_free(q) == 0 and L.bh_free(r) == 0 and L.bh_free(q) != 0
+
+
+def _free_bytes(bh):
+    hip = C.CDLL(bh._lib.LIB_PATH)  # the runtime's own symbols, through the library's dependency on it
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.gpu
+def test_trim_gives_back(bh):
+    """What the library keeps goes back on request: freed blocks, and the block paths' buffers of every thread,
+    one that lives on included; later calls work as before."""
+    import threading
+
+    n, kl, ku = 200000, 4, 4
+    h = np.ones((2 * kl + ku + 1, n), order="F")
+    h[kl + ku] = 40
+
+    def factor():
+        d, p, info = bh.DeviceArray.from_numpy(h), bh.DeviceArray((n,), np.int64), C.c_int64(-1)
+        bh._lib.call("bh_dgbtrf", n, n, kl, ku, d.ptr, 2 * kl + ku + 1, p.ptr, C.byref(info))
+        assert info.value == 0
+        return d.numpy()
+
+    first = factor()
+    bh.trim()
+    base = _free_bytes(bh)
+    a = bh.DeviceArray((64 << 20,), np.uint8)
+    a.free()
+    assert _free_bytes(bh) <= base - (64 << 20)
+    go, done, out = threading.Event(), threading.Event(), []
+
+    def other():
+        out.append(factor())
+        done.set()
+        go.wait(60)
+        out.append(factor())
+
+    t = threading.Thread(target=other)
+    t.start()
+    assert done.wait(60)
+    held = base - _free_bytes(bh)
+    assert held >= (64 << 20) + n * (2 * kl + ku + 1) * 8  # the block, the thread's copies of the matrix
+    bh.trim()
+    assert base - _free_bytes(bh) <= 8 << 20
+    go.set()
+    t.join(60)
+    assert len(out) == 2 and all(o.tobytes() == first.tobytes() for o in out)
