@@ -217,7 +217,9 @@ void *cut_alloc(size_t bytes, hipStream_t st) {
     bool ok = true;
     if (c->p && (c->dev != dev || c->bytes < bytes))
         ok = cut_release(*c);
-    else if (c->p && c->st != st)
+    else if (c->p)
+        // also on what looks like the same stream: it may be a new one at the
+        // handle of a destroyed one whose work still runs
         ok = hipStreamWaitEvent(st, c->done, 0) == hipSuccess;
     if (ok && c->done && c->dev != dev) {
         (void)hipEventDestroy(c->done);

@@ -295,3 +295,36 @@ def test_other_stream_captured(bh, monkeypatch):
     x = bh.DeviceArray.from_numpy(b)
     solve(x, [])  # the kernels loaded before the capture
     _same(*_both(monkeypatch, run))
+
+
+def test_stream_destroyed_and_another_created(bh, monkeypatch):
+    """Solves on streams that are destroyed right after them, before their work has ended; a new stream may have
+    the old one's handle, and its solve takes the same buffer: behind that work all the same."""
+    monkeypatch.delenv("BANDEDHIP_CUT", raising=False)
+    hip = C.CDLL(bh._lib.LIB_PATH)
+    n, k = 400003, 5
+    rng = np.random.default_rng(5)
+    A = bh.DeviceArray.from_numpy(_triangle(rng, n, k, True, np.float64, "dominant"))
+    b = [rng.standard_normal(n) for _ in range(6)]
+
+    def solve(x):
+        bh._lib.call("bh_dtbsv", b"U", b"N", b"N", n, k, A.ptr, k + 1, x.ptr, 1)
+
+    want = [bh.DeviceArray.from_numpy(v) for v in b]
+    for x in want:
+        solve(x)
+        bh.sync()
+    got = [bh.DeviceArray.from_numpy(v) for v in b]
+    try:
+        for x in got:
+            s = C.c_void_p()
+            assert hip.hipStreamCreateWithFlags(C.byref(s), C.c_uint(1)) == 0
+            bh._lib.call("bh_set_stream", s)
+            solve(x)
+            bh._lib.call("bh_set_stream", None)
+            assert hip.hipStreamDestroy(s) == 0
+    finally:
+        bh._lib.call("bh_set_stream", None)
+    assert hip.hipDeviceSynchronize() == 0
+    for g, w in zip(got, want):
+        _same((g.numpy(),), (w.numpy(),))
