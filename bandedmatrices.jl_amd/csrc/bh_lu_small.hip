@@ -426,37 +426,37 @@ int batch_autotune(bh_batch_plan *p, const T *AB, const T *B, double *best_ms) {
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
     const int wpb[] = {1, 2, 4};
-    const int mult[] = {1, 2, 4, 8};
+    const int mult[] = {1, 2, 4, 8, 12, 16};  // waves per CU: up to the four per SIMD of the default
     const int kinds[] = {0, 2};
     double best = 1e300;
-    int bw = p->waves_per_block, bb = p->blocks, bk = p->order_kind;
-    for (int kind : kinds) {
-        for (int w : wpb) {
-            for (int mu : mult) {
-                p->waves_per_block = w;
-                p->blocks = std::max(1, p->cus * mu / w);
-                if (plan_set_order(p, kind) != BH_OK) continue;
-                float ms_sum = 0.f;
-                for (int rep = 0; rep < 2; ++rep) {
-                    (void)hipMemcpyAsync(ab2, AB, sizeof(T) * p->ab_elems, hipMemcpyDeviceToDevice, s);
-                    (void)hipMemcpyAsync(b2, B, sizeof(T) * p->vec_elems, hipMemcpyDeviceToDevice, s);
-                    (void)hipEventRecord(e0, s);
-                    batch_launch<T>(p, ab2, b2, ip2, inf2, s);
-                    (void)hipEventRecord(e1, s);
-                    (void)hipEventSynchronize(e1);
-                    float ms = 0.f;
-                    (void)hipEventElapsedTime(&ms, e0, e1);
-                    if (rep > 0) ms_sum += ms;
-                }
-                if (ms_sum < best) {
-                    best = ms_sum;
-                    bw = w;
-                    bb = p->blocks;
-                    bk = kind;
-                }
-            }
+    const int w0 = p->waves_per_block, b0 = p->blocks, k0 = p->order_kind;
+    int bw = w0, bb = b0, bk = k0;
+    auto trial = [&](int w, int blocks, int kind) {
+        p->waves_per_block = w;
+        p->blocks = blocks;
+        if (plan_set_order(p, kind) != BH_OK) return;
+        float ms = 0.f;
+        for (int rep = 0; rep < 2; ++rep) {
+            (void)hipMemcpyAsync(ab2, AB, sizeof(T) * p->ab_elems, hipMemcpyDeviceToDevice, s);
+            (void)hipMemcpyAsync(b2, B, sizeof(T) * p->vec_elems, hipMemcpyDeviceToDevice, s);
+            (void)hipEventRecord(e0, s);
+            batch_launch<T>(p, ab2, b2, ip2, inf2, s);
+            (void)hipEventRecord(e1, s);
+            (void)hipEventSynchronize(e1);
+            (void)hipEventElapsedTime(&ms, e0, e1);
         }
-    }
+        if (ms < best) {
+            best = ms;
+            bw = w;
+            bb = blocks;
+            bk = kind;
+        }
+    };
+    // the schedule the plan has comes first: only a faster one takes its place
+    trial(w0, b0, k0);
+    for (int kind : kinds)
+        for (int w : wpb)
+            for (int mu : mult) trial(w, std::max(1, p->cus * mu / w), kind);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     cleanup();

@@ -125,3 +125,34 @@ def test_batched_schedule_is_fixed_while_a_graph_exists(bh, oracle):
     bt.solve()
     _check(oracle, bt, n, kl, ku, AB, B)
     bt.close()
+
+
+def test_batched_autotune_never_slows_a_plan_down(bh):
+    """The schedule a plan has is timed first and every width of the default is among the candidates: what
+    autotune leaves is no slower than the default (medians, a fifth allowed for noise), and a poor one is replaced."""
+    n, kl, ku, bands, rhs = _batch(bh, np.float64, nsys=4096, seed=6, nmin=100, nmax=1000,
+                                   classes=((1, 1), (2, 2), (4, 3), (8, 8)))
+    bt = bh.BatchedGBSV(n, kl, ku)
+    AB, B = bt.pack(bands, rhs)
+
+    def median():
+        t, ms = bh.Timer(), []
+        for _ in range(7):
+            bt.upload(AB, B)
+            t.start()
+            bt.solve()
+            t.stop()
+            ms.append(t.elapsed_ms())
+        return sorted(ms)[3]
+
+    default = median()
+    bt.upload(AB, B)
+    best = bt.autotune()
+    tuned = median()
+    print("default", default, "autotuned", tuned, bt.schedule())
+    assert tuned <= 1.2 * default and best <= 1.2 * default
+    bt.schedule(order=0, waves_per_block=1, blocks=16)
+    bt.upload(AB, B)
+    bt.autotune()
+    assert median() <= 1.2 * default
+    bt.close()
