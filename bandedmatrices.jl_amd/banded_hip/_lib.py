@@ -26,6 +26,7 @@ SIGNATURES: dict[str, tuple] = {
     "bh_malloc": (C.c_int, [C.POINTER(vp), C.c_size_t]),
     "bh_free": (C.c_int, [vp]),
     "bh_trim": (C.c_int, []),
+    "bh_cut_verdict": (C.c_int, [C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "bh_memcpy_htod": (C.c_int, [vp, vp, C.c_size_t]),
     "bh_memcpy_dtoh": (C.c_int, [vp, vp, C.c_size_t]),
     "bh_memcpy_dtod": (C.c_int, [vp, vp, C.c_size_t]),

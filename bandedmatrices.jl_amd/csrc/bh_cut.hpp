@@ -38,6 +38,10 @@ void cut_free(void *p, hipStream_t st);
 // False when the environment says BANDEDHIP_CUT=off or a caller that may not
 // allocate has switched it off for this thread.
 bool cut_enabled();
+// For bh_cut_verdict: a call that can run by blocks begins (nothing tried yet);
+// blocks are launched whose verdict will stand in flags, in a buffer of cut_alloc.
+void cut_begin();
+void cut_note(const int *flags, hipStream_t st);
 struct CutOff {  // no cutting on this thread while one of these lives
     CutOff();
     ~CutOff();

@@ -294,6 +294,7 @@ static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 
             cut_free(ws, st);
             return r == -1 ? BH_OK : r;  // -1: the kernel does not take this band
         }
+        cut_note(flags, st);
         hipLaunchKernelGGL(lu_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, kv, (int)up16(kv), flags);
         hipLaunchKernelGGL(lu_cut_commit<T>, dim3(gx, g.p), dim3(256), 0, st, cut, ab, ldab, ipiv);
         hipError_t e = hipGetLastError();
@@ -350,6 +351,7 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
         kind = kLuBlk;
     void *ws = nullptr;
     LuCut<T> seq{};
+    cut_begin();
     if (m == n && kind != kLuNone) {
         const int cs = gbtrf_cut<T>(kind, n, kl, ku, ab, ldab, ipiv, &ws, &seq);
         if (cs) return cs;

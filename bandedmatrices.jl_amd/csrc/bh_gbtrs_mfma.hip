@@ -695,6 +695,7 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
     const CutGeom gl = trs_geom<T>(L.np, kl, grid.x), gu = trs_geom<T>(L.np, kl + ku, grid.x);
     SweepCut<T> cut{};
     char *ws = nullptr;
+    cut_begin();
     if (gl.p > 0 && gu.p > 0 && 16 * n * (i64)sizeof(T) < kQOob && cut_enabled()) {
         auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
         const i64 cols = 16 * (i64)grid.x;  // whole groups of 16 columns
@@ -716,6 +717,7 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
             hipLaunchKernelGGL(sweep_check<T>, dim3(gu.p - 1, grid.x), dim3(256), 0, st, (const T *)snu, cu, flags);
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n,
                                (const T *)Z, B, 1, ldb, (const int *)flags);
+            cut_note(flags, st);
             cut.flags = flags;
         }
     }

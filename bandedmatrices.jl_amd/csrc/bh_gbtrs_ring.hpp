@@ -429,6 +429,7 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
     const CutGeom gu = sweep_geom<T>(n, kd, nrhs, NB), gl = sweep_geom<T>(n - 1, kl, nrhs, NF);
     char *ws = nullptr;
     int *flags = nullptr;
+    if (how != 0) cut_begin();
     if (how != 0 && gu.p > 0 && (kl == 0 || gl.p > 0) && cut_enabled()) {
         auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
         const size_t by = al((size_t)n * nrhs * sizeof(T));
@@ -459,6 +460,7 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
             }
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n,
                                in, B, 1, ldb, (const int *)flags);
+            cut_note(flags, st);
             seq.cut.flags = flags;
         }
     }

@@ -288,6 +288,7 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
     // blocks agreed.
     PbCut<T> cut{};
     char *ws = nullptr;
+    cut_begin();
     const CutGeom g = pb_cut_geom<T>(n, kd);
     // an upper Cholesky with kd <= 8: one lane per block (0.32 ms with a
     // workgroup per block at n = 65536, kd = 8, FP64; 0.13 with a lane)
@@ -305,6 +306,7 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
                 cut_free(ws, st);
                 return r;
             }
+            cut_note(flags, st);
             cut.flags = flags;
             e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
         }
@@ -322,6 +324,7 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
             hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, (int)kd, (int)up, flags);
             hipLaunchKernelGGL(pb_cut_commit<T>, dim3((unsigned)imin(16, cdiv(g.L * H, 256)), g.p), dim3(256), 0, st,
                                cut, (int)kd, ab, ldab);
+            cut_note(flags, st);
             e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
             cut.g.p = 0;
         }

@@ -123,6 +123,15 @@ struct CutBufs {
     CutBuf b[4];
     unsigned long long clock = 0;
     int off = 0;
+    // the last call that could run by blocks: how often blocks were launched,
+    // where its verdict stands (null once the buffer has gone back) or what it was
+    int tries = 0, known[2] = {1, 0};
+    const int *flags = nullptr;
+    hipStream_t flags_st = nullptr;
+    bool holds_flags(const CutBuf &c) const {
+        const char *f = (const char *)flags, *p = (const char *)c.p;
+        return f && p && f >= p && f < p + c.bytes;
+    }
     CutBufs() {
         std::lock_guard<std::mutex> all(g_cut_mutex);
         g_cut_all.push_back(this);
@@ -147,8 +156,14 @@ static void cut_release_idle() {
     std::lock_guard<std::mutex> all(g_cut_mutex);
     for (CutBufs *t : g_cut_all) {
         std::lock_guard<std::mutex> lock(t->m);
-        for (CutBuf &c : t->b)
-            if (!c.busy) (void)cut_release(c);
+        for (CutBuf &c : t->b) {
+            if (c.busy || !c.p) continue;
+            const bool noted = t->holds_flags(c);
+            if (cut_release(c) && noted) {
+                t->flags = nullptr;
+                t->tries = 0;
+            }
+        }
     }
 }
 
@@ -188,6 +203,19 @@ bool cut_enabled() {
     if (g_cut.off > 0) return false;
     const char *e = getenv("BANDEDHIP_CUT");
     return !(e && !strcmp(e, "off"));
+}
+
+void cut_begin() {
+    std::lock_guard<std::mutex> lock(g_cut.m);
+    g_cut.tries = 0;
+    g_cut.flags = nullptr;
+}
+
+void cut_note(const int *flags, hipStream_t st) {
+    std::lock_guard<std::mutex> lock(g_cut.m);
+    ++g_cut.tries;
+    g_cut.flags = flags;
+    g_cut.flags_st = st;
 }
 
 void *cut_alloc(size_t bytes, hipStream_t st) {
@@ -252,6 +280,10 @@ void cut_free(void *p, hipStream_t st) {
         if (!c.busy || c.p != p) continue;
         if (c.bytes > kCutKeep || hipEventRecord(c.done, st) != hipSuccess) {
             const RelaxedCapture relaxed;
+            if (g_cut.holds_flags(c)) {
+                (void)hipMemcpyAsync(g_cut.known, g_cut.flags, sizeof g_cut.known, hipMemcpyDeviceToHost, st);
+                g_cut.flags = nullptr;
+            }
             (void)hipStreamSynchronize(st);
             (void)hipFree(c.p);
             c.p = nullptr;
@@ -332,6 +364,20 @@ int bh_free(void *dptr) {
 
 int bh_trim(void) {
     release_kept();
+    return BH_OK;
+}
+
+int bh_cut_verdict(int *verdict_host, int *tries_host) {
+    BH_ARG(verdict_host != nullptr, 1);
+    std::lock_guard<std::mutex> lock(g_cut.m);
+    *verdict_host = 0;
+    if (tries_host) *tries_host = g_cut.tries;
+    if (g_cut.tries == 0) return BH_OK;
+    if (g_cut.flags) {
+        BH_HIP(hipMemcpyAsync(g_cut.known, g_cut.flags, sizeof g_cut.known, hipMemcpyDeviceToHost, g_cut.flags_st));
+        BH_HIP(hipStreamSynchronize(g_cut.flags_st));
+    }
+    *verdict_host = g_cut.known[0] ? 2 : (g_cut.known[1] ? 3 : 1);
     return BH_OK;
 }
 

@@ -248,6 +248,7 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
     auto kern = tbsv_ring<T, MODE, NW, PFD>;
     SweepCut<T> cut{};
     char *ws = nullptr;
+    cut_begin();
     const CutGeom g = sweep_geom<T>(n, k, nrhs, NW);
     // 'N' with k <= 16: one lane per block (bh_tbsv_lane.hpp), where the blocks
     // are the shorter (L + W steps of 0.1-0.2 us against 0.3)
@@ -278,6 +279,7 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
             }
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), nrhs), dim3(256), 0, st, n, (const T *)y,
                                x, incx, ldx, (const int *)flags);
+            cut_note(flags, st);
             cut.flags = flags;
             cut.g.p = 0;
         }

@@ -54,6 +54,14 @@ int bh_free(void *dptr);
  * call uses just then.  Waits for the work that used them.  It happens by
  * itself when an allocation of the library finds none left. */
 int bh_trim(void);
+/* What became of this thread's last factorisation or solve of the kind that can
+ * run by blocks (gbtrf, pbtrf, sbldlt, each sweep of tbsv and of what is built
+ * on it, gbtrs, gbtrs_part, gbtrs_blocked): *verdict_host is 1 when the blocks
+ * agreed and are the result, 2 when the matrix was not tried (its sampled
+ * diagonal does not dominate), 3 when they differed and the sequential kernels
+ * ran, 0 when there were no blocks (or their memory has been given back).
+ * *tries_host (may be NULL): how often blocks were launched.  Waits for that call. */
+int bh_cut_verdict(int *verdict_host, int *tries_host);
 int bh_memcpy_htod(void *dst, const void *src_host, size_t bytes);
 int bh_memcpy_dtoh(void *dst_host, const void *src, size_t bytes);
 int bh_memcpy_dtod(void *dst, const void *src, size_t bytes);
