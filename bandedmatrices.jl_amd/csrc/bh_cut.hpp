@@ -94,10 +94,24 @@ struct PbLane {
     int p, L, W;  // blocks, own columns, lead-in
 };
 
-// Gate: 256 columns spread over the matrix, 16 lanes to a column (64 columns
-// and a wave to each where they are longer than 64 entries: 42 -> 19 us at
+// Gate: 256 columns spread over the matrix, 16 lanes to a column (64 columns,
+// a wave to each, where they are longer than 64 entries: 42 -> 19 us at
 // 385 and 129 entries); closed when more than a quarter of them have num/4 times the sum of |a| off the
 // diagonal above |a_jj|.  One workgroup, so it writes both flags itself.
+// rate > 0 (a symmetric matrix of which s1 holds one triangle): closed also
+// when the mean over the sampled columns of
+//     -sum over the stored entries at distance t of s^t a_t (z^t + z^-t) / a_jj,  z = 2^-rate,
+// is above 1 for s = 1 or s = -1.  A constant band with those coefficients
+// forgets by the factor z per step (twice per step in its factorisation) where
+// that sum is 1, in the mode that is constant or alternates; above it, too
+// slowly for the lead-in.  Coefficients of random signs average out, as they do
+// in the chain.  Dominance alone does not tell: the second difference (2, -1)
+// and the five-point Laplacian (4, -1, -1) are at twice the sum of the stored
+// half, and never agree; they stand at 1.02 to 1.35 here (kd = 1 .. 64, FP32
+// and FP64).  Random, constant and Laplacian bands over diagonals of 1 to 2
+// times the other entries, simulated: what the test closes never agrees within
+// the lead-in; of what it leaves open, wide Laplacians at 1.25 to 3 times
+// dominance (kd = 64) do not agree either and pay for the trial.
 // A set of entries of a column: rows r0 .. r0+h-1 of the band array, the
 // diagonal in row d (with `unit` it counts as 1); h = 0: no second set.
 struct CutSet {
@@ -105,8 +119,9 @@ struct CutSet {
 };
 template <typename T>
 __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, CutSet s1, CutSet s2, int num,
-                                                 int *flags) {
+                                                 float rate, int *flags) {
     __shared__ int weak[2];
+    __shared__ float part[2][64];
     if (threadIdx.x < 2) weak[threadIdx.x] = 0;
     __syncthreads();
     const int lanes = s1.h > 64 ? 64 : 16, cols = 1024 / lanes, samples = 4 * cols;
@@ -118,22 +133,56 @@ __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld
         for (int off = lanes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
         return T(4) * (s.unit ? T(1) : dabs(col[s.d])) >= T(num) * t;
     };
+    float mean[2] = {0.0f, 0.0f};
+    auto coherent = [&](const T *col, i64 c) {  // slots outside the matrix hold anything
+        T even = T(0), odd = T(0);
+        for (int r = q; r < s1.h; r += lanes) {
+            const int dist = s1.r0 + r - s1.d;
+            if (dist == 0 || c + dist < 0 || c + dist >= n) continue;
+            const float z = exp2f(rate * (float)dist);
+            const T t = col[s1.r0 + r] * T(z + 1.0f / z);
+            (dist & 1 ? odd : even) += t;
+        }
+        for (int off = lanes / 2; off > 0; off >>= 1) {
+            even += __shfl_xor(even, off, 64);
+            odd += __shfl_xor(odd, off, 64);
+        }
+        mean[0] -= (float)((even + odd) / col[s1.d]);
+        mean[1] -= (float)((even - odd) / col[s1.d]);
+    };
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-        const i64 c = ((i64)(cols * it + g) * n + n / 2) / samples;
+        // the golden section spreads the samples evenly without a stride, which a
+        // grid's rows could be in step with
+        const i64 c = (i64)(((unsigned long long)((unsigned)(cols * it + g + 1) * 2654435769u) * (unsigned)n) >> 32);
         const T *col = a + c * ld;
         m1 += !strong(col, s1);
         if (s2.h) m2 += !strong(col, s2);
+        if (rate > 0.0f) coherent(col, c);
     }
     if (q == 0) {
         atomicAdd(&weak[0], m1);
         atomicAdd(&weak[1], m2);
+        part[0][g] = mean[0];
+        part[1][g] = mean[1];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        flags[0] = weak[0] > samples / 4 || weak[1] > samples / 4;
+        float t0 = 0.0f, t1 = 0.0f;
+        for (int i = 0; i < cols; ++i) {
+            t0 += part[0][i];
+            t1 += part[1][i];
+        }
+        flags[0] = weak[0] > samples / 4 || weak[1] > samples / 4 || !(t0 <= (float)samples) || !(t1 <= (float)samples);
         flags[1] = 0;
     }
+}
+
+// The gate's rate for a lead-in of W steps: the chain forgets twice the rate's
+// bits a step, and all but the last few of the type's must be gone after W.
+template <typename T>
+inline float cut_rate(i64 W) {
+    return (sizeof(T) == 8 ? 48.0f : 24.0f) / (2.0f * (float)W);
 }
 
 // ---------------------------------------------------------------- solves

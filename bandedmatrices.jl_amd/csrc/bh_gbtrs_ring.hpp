@@ -441,7 +441,7 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
             T *Y = (T *)ws, *Z = (T *)(ws + by), *snu = (T *)(ws + 2 * by), *snl = (T *)(ws + 2 * by + su);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, ab, ld, (int)n,
                                CutSet{0, (int)kd + 1, (int)kd, 0}, CutSet{(int)kd, kl ? (int)kl + 1 : 0, (int)kd, 1},
-                               5, flags);
+                               5, 0.0f, flags);
             const T *in = B;
             i64 ldin = ldb;
             T *out = Y;

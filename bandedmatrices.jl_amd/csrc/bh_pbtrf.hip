@@ -284,8 +284,8 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
     hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // By blocks where |a_jj| is at least 1.75 times the sum of its stored
     // row or column (half of the off-diagonal entries: plain dominance is 2
-    // on average); behind them the whole chain, which does nothing where the
-    // blocks agreed.
+    // on average) and the gate's rate test leaves room for the lead-in; behind
+    // them the whole chain, which does nothing where the blocks agreed.
     PbCut<T> cut{};
     char *ws = nullptr;
     cut_begin();
@@ -300,7 +300,7 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
         if (ws) {
             int *flags = (int *)(ws + bo + bs);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, (int)kd, 0}, CutSet{}, 7, flags);
+                               CutSet{0, (int)H, (int)kd, 0}, CutSet{}, 7, cut_rate<T>(gl.W), flags);
             const int r = pbtrf_lane_run<T>(gl, n, kd, ab, ldab, (T *)ws, (T *)(ws + bo), flags, st);
             if (r != BH_OK) {
                 cut_free(ws, st);
@@ -318,7 +318,7 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
             int *flags = (int *)(ws + bo + bi);
             cut = PbCut<T>{g, flags, (T *)ws, (i64 *)(ws + bo)};
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, flags);
+                               CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, cut_rate<T>(g.W), flags);
             hipLaunchKernelGGL(kern, dim3(g.p), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, (T *)nullptr,
                                (i64)0, (i64 *)nullptr, (int)B, cut);
             hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, (int)kd, (int)up, flags);

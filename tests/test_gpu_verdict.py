@@ -220,3 +220,33 @@ def test_blocked_solve(bh, dtype, n, kl, ku, nrhs):
         f, piv = _gbtrf(bh, _dominant(n, kl, ku, dtype, shift), n, kl, ku)
         bh._lib.call(f"bh_{p}gbtrs_blocked", n, kl, ku, nrhs, f.ptr, 2 * kl + ku + 1, piv.ptr, b.ptr, n, ws.ptr, nb.value)
         assert verdict(bh)[0] == want
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("ldl", [False, True])
+@pytest.mark.parametrize("n,kd", [(5120, 64), (65536, 8), (20000, 20), (10001, 1), (1999, 1)])
+def test_laplacians_are_not_tried(bh, dtype, uplo, ldl, n, kd):
+    """The second difference and the five-point Laplacian never forget where a chain began, although their diagonal is
+    twice the sum of the stored half: the gate refuses them.  With 16 times the diagonal it does not.  The slots
+    outside the matrix hold NaN."""
+    up = uplo == "U"
+    A = np.zeros((kd + 1, n))
+    if kd > 1:
+        A[0 if up else kd] = -1
+    A[kd - 1 if up else 1] = -1
+    if kd > 1:  # a grid's rows are not coupled end to end
+        A[kd - 1 if up else 1, (0 if up else kd - 1)::kd] = 0
+    for c in range(kd):
+        if up:
+            A[:kd - c, c] = np.nan
+        else:
+            A[c + 1:, n - 1 - c] = np.nan
+    for scale, want in ((1, REFUSED), (16, AGREED)):
+        A[kd if up else 0] = scale * (2 if kd == 1 else 4)
+        x, info = bh.DeviceArray.from_numpy(np.asfortranarray(A.astype(dtype))), C.c_int64(0)
+        if ldl:
+            bh._lib.call(f"bh_{FP[dtype]}sbldlt", uplo.encode(), n, kd, x.ptr, kd + 1)
+        else:
+            bh._lib.call(f"bh_{FP[dtype]}pbtrf", uplo.encode(), n, kd, x.ptr, kd + 1, C.byref(info))
+        assert info.value == 0 and verdict(bh)[0] == want, scale
