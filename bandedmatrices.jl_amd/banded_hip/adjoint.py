@@ -49,7 +49,8 @@ def mul_pullback(A: BandedMatrix, x0: DeviceArray, ybar: DeviceArray):
 def loss_and_grad(A: BandedMatrix, b: DeviceArray, w: DeviceArray, x0: DeviceArray, method: str = "auto"):
     """L = w' A^{-1} b + 1/2 ||A x0||^2 with its gradient: returns (L, dA, db, x).
     method: the two solves' method (ldiv_'s "auto" -- partitioned from n = 4096
-    on --, "exact" or "partitioned").
+    on, whatever the factors --, "exact", which is a little faster where they are
+    dominant and far slower where not, or "partitioned").
 
     Forward: band LU, 'N' solve, gbmv.  Backward: 'T' solve with the same
     factors and pivots, then one fused band kernel

@@ -161,9 +161,12 @@ def ldiv_(F, B: DeviceArray, method: str = "exact") -> DeviceArray:
     of a BandedMatrix (UpperTriangular(A) etc., solved with tbsv).
 
     method="exact": LAPACK's gbtrs operation order on the GPU, bit for bit.
-    method="partitioned": the rows split into blocks solved at once across the
-    GPU (bh_?gbtrs_part, kl <= 31 and kl + ku <= 63): equal to rounding; falls
-    back to the exact solve outside that range.
+    Dominant factors are solved by blocks at once, which makes it the fastest
+    method for them (no wait on the host); others as one chain.
+    method="partitioned": what is not dominant split into blocks solved at once
+    by their transfer matrices too (bh_?gbtrs_part, kl <= 31 and kl + ku <= 63):
+    equal to rounding; dominant factors as "exact", some 10-30 us behind it;
+    falls back to the exact solve outside that range.
     method="blocked": 'N' only, panels of 32 rows on the matrix cores
     (bh_?gbtrs_blocked): equal to rounding; for wide bands; falls back to the
     exact solve for 'T' or outside its range.

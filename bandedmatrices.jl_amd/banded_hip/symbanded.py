@@ -170,7 +170,8 @@ def cholesky_ldiv_(F: BandedCholesky, B: DeviceArray, method: str = "exact") -> 
     upper factor U (its (k+1) x n band is LAPACK's AB layout of a band LU with
     kl = 0, ku = k) with k <= 63 is solved as U^T y = B, U x = y by the
     partitioned band solve (bh_?gbtrs_part, identity pivots; equal to rounding);
-    a lower factor or a wider band falls back to the exact solve."""
+    a lower factor or a wider band falls back to the exact solve, which is the
+    faster one where the factor's diagonal dominates (by blocks)."""
     n = F.shape[0]
     if B.shape[0] != n:
         raise DimensionMismatch(f"matrix A has dimensions {F.shape}, but right hand side B has {B.shape}")

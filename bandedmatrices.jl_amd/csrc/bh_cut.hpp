@@ -35,6 +35,15 @@ constexpr size_t kCutKeep = size_t(2) << 30;
 constexpr size_t kCutMax = size_t(8) << 30;
 void *cut_alloc(size_t bytes, hipStream_t st);
 void cut_free(void *p, hipStream_t st);
+// For a caller that waits for a verdict before it goes on: kCutWords words of
+// this thread's pinned host memory, -1 each, into which kernels write values
+// >= 0 (nullptr: none to be had), and a wait for one of them: its value, or -1
+// when the stream has ended without it.  (A wait through a copy to the host
+// left the device idle for 50 us before the next kernel, through an event some
+// 15; the word is there in a few.)
+constexpr int kCutWords = 4;
+int *cut_host_words();
+int cut_poll(const int *word, hipStream_t st);
 // False when the environment says BANDEDHIP_CUT=off or a caller that may not
 // allocate has switched it off for this thread.
 bool cut_enabled();
@@ -60,6 +69,11 @@ struct CutGeom {
 __device__ __forceinline__ bool cut_closed(const int *flags) { return __hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; }
 __device__ __forceinline__ bool cut_failed(const int *flags) {
     return cut_closed(flags) || __hip_atomic_load(flags + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
+// a word of the host's
+__device__ __forceinline__ void cut_tell(int *word, int v) {
+    if (word) __hip_atomic_store(word, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __device__ __forceinline__ bool cut_differ(double a, double b) {
@@ -97,7 +111,8 @@ struct PbLane {
 // Gate: 256 columns spread over the matrix, 16 lanes to a column (64 columns,
 // a wave to each, where they are longer than 64 entries: 42 -> 19 us at
 // 385 and 129 entries); closed when more than a quarter of them have num/4 times the sum of |a| off the
-// diagonal above |a_jj|.  One workgroup, so it writes both flags itself.
+// diagonal above |a_jj|.  One workgroup, so it writes both flags itself (and the
+// first one to a word of the host's, where there is one).
 // rate > 0 (a symmetric matrix of which s1 holds one triangle): closed also
 // when the mean over the sampled columns of
 //     -sum over the stored entries at distance t of s^t a_t (z^t + z^-t) / a_jj,  z = 2^-rate,
@@ -119,7 +134,7 @@ struct CutSet {
 };
 template <typename T>
 __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, CutSet s1, CutSet s2, int num,
-                                                 float rate, int *flags) {
+                                                 float rate, int *flags, int *host) {
     __shared__ int weak[2];
     __shared__ float part[2][64];
     if (threadIdx.x < 2) weak[threadIdx.x] = 0;
@@ -173,8 +188,11 @@ __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld
             t0 += part[0][i];
             t1 += part[1][i];
         }
-        flags[0] = weak[0] > samples / 4 || weak[1] > samples / 4 || !(t0 <= (float)samples) || !(t1 <= (float)samples);
+        const int closed =
+            weak[0] > samples / 4 || weak[1] > samples / 4 || !(t0 <= (float)samples) || !(t1 <= (float)samples);
+        flags[0] = closed;
         flags[1] = 0;
+        cut_tell(host, closed);
     }
 }
 
@@ -200,11 +218,12 @@ struct SweepCut {
     }
 };
 
-// The memory of a solve by blocks alone (nullptr: none ran) and its verdict,
-// freed by whoever asked for it after reading the flags.
+// The memory of a solve by blocks alone (nullptr: it is not to be had that way)
+// and its verdict, freed by whoever asked for it.
 struct RingCutWs {
     void *ws = nullptr;
-    const int *flags = nullptr;
+    int *flags = nullptr;
+    int *host = nullptr;  // [0]: whether the gate is closed; [1]: whether the blocks failed; two more for the caller
 };
 
 // cnt entries per window; grid (p - 1, nrhs)
@@ -219,11 +238,13 @@ __global__ void __launch_bounds__(256) sweep_check(const T *__restrict__ snap, i
     if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(flags + 1, 1);
 }
 
-// the blocks' results (n x nrhs, contiguous) to the caller's vectors
+// the blocks' results (n x nrhs, contiguous) to the caller's vectors; host: told whether they failed
 template <typename T>
 __global__ void __launch_bounds__(256) sweep_commit(int n, const T *__restrict__ y, T *__restrict__ x, int incx,
-                                                    i64 ldx, const int *flags) {
-    if (cut_failed(flags)) return;
+                                                    i64 ldx, const int *flags, int *host) {
+    const bool failed = cut_failed(flags);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) cut_tell(host, failed);
+    if (failed) return;
     const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
     if (i < n) x[(i64)blockIdx.y * ldx + i * incx] = y[(i64)blockIdx.y * n + i];
 }

@@ -286,7 +286,7 @@ static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 
         int *flags = (int *)(ws + ba + bp + bi);
         const LuCut<T> cut{g, flags, (T *)ws, (i64 *)(ws + ba), (i64 *)(ws + ba + bp), H, (int)kl};
         hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                           CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, 0.0f, flags);
+                           CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, 0.0f, flags, (int *)nullptr);
         const unsigned gx = (unsigned)imin(64, cdiv((i64)g.span() * H, 1024));
         hipLaunchKernelGGL(lu_cut_copy<T>, dim3(gx, g.p), dim3(256), 0, st, cut, (const T *)ab, ldab, kv);
         const int r = lu_kernel_launch<T>(kind, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);

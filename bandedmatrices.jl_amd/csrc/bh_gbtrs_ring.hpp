@@ -414,11 +414,12 @@ __global__ void __launch_bounds__(64) gbtrs_t_ring(int n, int kl, int ku, const 
 
 // Both sweeps with one kernel.  `how`: 0 the whole system; 1 by blocks if it
 // can be cut, and behind them the whole system, which does nothing where they
-// agreed; 2 the blocks alone, *cw telling whether they ran (for a caller with
-// another fallback).  Gate: U's columns at 1.25 times the rest of the column,
-// L's multipliers summing to less than 0.8.  Measured FP64 1 RHS against the
-// whole sweeps: n = 262144, (16,16) the two solves of a gradient 5.3 -> 0.7 ms
-// (60.7 and 100 ms as whole sweeps, 2.6 and 2.7 partitioned).
+// agreed; for a caller with another fallback, that waits for the verdicts: 2
+// the gate alone (*cw: the memory, or none), 3 the blocks behind it.  Gate: U's
+// columns at 1.25 times the rest of the column, L's multipliers summing to less
+// than 0.8.  Measured FP64 1 RHS against the whole sweeps: n = 262144, (16,16)
+// the two solves of a gradient 5.3 -> 0.7 ms (60.7 and 100 ms as whole sweeps,
+// 2.6 and 2.7 partitioned).
 template <typename T, int NF, int NB, class K>
 int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ld, const i64 *ipiv, T *B,
              i64 ldb, hipStream_t st, RingCutWs *cw) {
@@ -427,50 +428,54 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
     RingWork<T> seq{3, B, B, ldb, ldb, SweepCut<T>{}};
     // the sweep with L has n-1 steps, the one with U n
     const CutGeom gu = sweep_geom<T>(n, kd, nrhs, NB), gl = sweep_geom<T>(n - 1, kl, nrhs, NF);
-    char *ws = nullptr;
-    int *flags = nullptr;
-    if (how != 0) cut_begin();
-    if (how != 0 && gu.p > 0 && (kl == 0 || gl.p > 0) && cut_enabled()) {
-        auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-        const size_t by = al((size_t)n * nrhs * sizeof(T));
-        const size_t su = al((size_t)gu.p * nrhs * 2 * 64 * NB * sizeof(T));
-        const size_t sl = kl ? al((size_t)gl.p * nrhs * 2 * 64 * NF * sizeof(T)) : 0;
-        ws = (char *)cut_alloc(2 * by + su + sl + 256, st);
+    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t by = al((size_t)n * nrhs * sizeof(T));
+    const size_t su = al((size_t)gu.p * nrhs * 2 * 64 * NB * sizeof(T));
+    const size_t sl = kl ? al((size_t)gl.p * nrhs * 2 * 64 * NF * sizeof(T)) : 0;
+    char *ws = how == 3 ? (char *)cw->ws : nullptr;
+    int *flags = how == 3 ? cw->flags : nullptr, *host = how == 3 ? cw->host : nullptr;
+    if (how == 1 || how == 2) cut_begin();
+    if ((how == 1 || how == 2) && gu.p > 0 && (kl == 0 || gl.p > 0) && cut_enabled()) {
+        if (how == 2) host = cut_host_words();
+        if (how == 1 || host) ws = (char *)cut_alloc(2 * by + su + sl + 256, st);
         if (ws) {
             flags = (int *)(ws + 2 * by + su + sl);
-            T *Y = (T *)ws, *Z = (T *)(ws + by), *snu = (T *)(ws + 2 * by), *snl = (T *)(ws + 2 * by + su);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, ab, ld, (int)n,
                                CutSet{0, (int)kd + 1, (int)kd, 0}, CutSet{(int)kd, kl ? (int)kl + 1 : 0, (int)kd, 1},
-                               5, 0.0f, flags);
-            const T *in = B;
-            i64 ldin = ldb;
-            T *out = Y;
-            for (int sweep = 1; sweep <= 2; ++sweep) {
-                const bool lower = trans == (sweep == 2);
-                if (lower && kl == 0) continue;
-                const CutGeom &g = lower ? gl : gu;
-                T *snap = lower ? snl : snu;
-                hipLaunchKernelGGL(kern, dim3((unsigned)nrhs, g.p), block, 0, st, (int)n, (int)kl, (int)ku, ab, ld, ipiv,
-                                   RingWork<T>{sweep, in, out, ldin, n, SweepCut<T>{g, flags, snap}});
-                hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, (unsigned)nrhs), dim3(256), 0, st, (const T *)snap,
-                                   64 * (lower ? NF : NB), flags);
-                in = out;
-                ldin = n;
-                out = Z;
-            }
-            hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n,
-                               in, B, 1, ldb, (const int *)flags);
+                               5, 0.0f, flags, host);
             cut_note(flags, st);
-            seq.cut.flags = flags;
         }
     }
-    if (how != 2)
+    if (ws && how != 2) {
+        T *Y = (T *)ws, *Z = (T *)(ws + by), *snu = (T *)(ws + 2 * by), *snl = (T *)(ws + 2 * by + su);
+        const T *in = B;
+        i64 ldin = ldb;
+        T *out = Y;
+        for (int sweep = 1; sweep <= 2; ++sweep) {
+            const bool lower = trans == (sweep == 2);
+            if (lower && kl == 0) continue;
+            const CutGeom &g = lower ? gl : gu;
+            T *snap = lower ? snl : snu;
+            hipLaunchKernelGGL(kern, dim3((unsigned)nrhs, g.p), block, 0, st, (int)n, (int)kl, (int)ku, ab, ld, ipiv,
+                               RingWork<T>{sweep, in, out, ldin, n, SweepCut<T>{g, flags, snap}});
+            hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, (unsigned)nrhs), dim3(256), 0, st, (const T *)snap,
+                               64 * (lower ? NF : NB), flags);
+            in = out;
+            ldin = n;
+            out = Z;
+        }
+        hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), (unsigned)nrhs), dim3(256), 0, st, (int)n, in,
+                           B, 1, ldb, (const int *)flags, host ? host + 1 : nullptr);
+        seq.cut.flags = flags;
+    }
+    if (how < 2)
         hipLaunchKernelGGL(kern, dim3((unsigned)nrhs), block, 0, st, (int)n, (int)kl, (int)ku, ab, ld, ipiv, seq);
     const hipError_t e = hipGetLastError();
-    if (how == 2 && e == hipSuccess)
-        *cw = RingCutWs{ws, flags};
-    else
+    if (how < 2 || (how == 2 && e != hipSuccess)) {
         cut_free(ws, st);
+        ws = nullptr;
+    }
+    if (how == 2) *cw = RingCutWs{ws, flags, host};
     return e == hipSuccess ? BH_OK : hip_fail(e, "kernel launch", __FILE__, __LINE__);
 }
 

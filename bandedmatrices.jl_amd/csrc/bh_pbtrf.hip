@@ -300,7 +300,8 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
         if (ws) {
             int *flags = (int *)(ws + bo + bs);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, (int)kd, 0}, CutSet{}, 7, cut_rate<T>(gl.W), flags);
+                               CutSet{0, (int)H, (int)kd, 0}, CutSet{}, 7, cut_rate<T>(gl.W), flags,
+                               (int *)nullptr);
             const int r = pbtrf_lane_run<T>(gl, n, kd, ab, ldab, (T *)ws, (T *)(ws + bo), flags, st);
             if (r != BH_OK) {
                 cut_free(ws, st);
@@ -318,7 +319,8 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
             int *flags = (int *)(ws + bo + bi);
             cut = PbCut<T>{g, flags, (T *)ws, (i64 *)(ws + bo)};
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, cut_rate<T>(g.W), flags);
+                               CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, cut_rate<T>(g.W), flags,
+                               (int *)nullptr);
             hipLaunchKernelGGL(kern, dim3(g.p), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, (T *)nullptr,
                                (i64)0, (i64 *)nullptr, (int)B, cut);
             hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, (int)kd, (int)up, flags);

@@ -128,6 +128,7 @@ struct CutBufs {
     int tries = 0, known[2] = {1, 0};
     const int *flags = nullptr;
     hipStream_t flags_st = nullptr;
+    int *host = nullptr;  // pinned
     bool holds_flags(const CutBuf &c) const {
         const char *f = (const char *)flags, *p = (const char *)c.p;
         return f && p && f >= p && f < p + c.bytes;
@@ -146,6 +147,7 @@ struct CutBufs {
             if (c.p) (void)hipFree(c.p);
             if (c.done) (void)hipEventDestroy(c.done);
         }
+        if (host) (void)hipHostFree(host);
     }
 };
 static thread_local CutBufs g_cut;
@@ -203,6 +205,32 @@ bool cut_enabled() {
     if (g_cut.off > 0) return false;
     const char *e = getenv("BANDEDHIP_CUT");
     return !(e && !strcmp(e, "off"));
+}
+
+int *cut_host_words() {
+    if (!g_cut.host) {
+        const RelaxedCapture relaxed;
+        if (hipHostMalloc((void **)&g_cut.host, kCutWords * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            g_cut.host = nullptr;
+            return nullptr;
+        }
+    }
+    for (int i = 0; i < kCutWords; ++i) g_cut.host[i] = -1;
+    return g_cut.host;
+}
+
+int cut_poll(const int *word, hipStream_t st) {
+    const RelaxedCapture relaxed;
+    for (;;) {
+        for (int i = 0; i < 256; ++i) {
+            const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+            if (v >= 0) return v;
+            __builtin_ia32_pause();
+        }
+        // (the word may come between the look at it and the stream's end)
+        if (hipStreamQuery(st) != hipErrorNotReady) return __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    }
 }
 
 void cut_begin() {

@@ -263,7 +263,7 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
             int *flags = (int *)(ws + by + bs);
             T *y = (T *)ws, *snap = (T *)(ws + by);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, a, lda, n,
-                               CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, 0.0f, flags);
+                               CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, 0.0f, flags, (int *)nullptr);
             if (gl.p > 0) {
                 const int r = tbsv_lane_run(gl, TbMode<MODE>::ASC, n, k, a, lda, x, incx, ldx, nrhs, unit, y, snap,
                                             flags, st);
@@ -278,7 +278,7 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
                 hipLaunchKernelGGL(sweep_check<T>, dim3(g.p - 1, nrhs), dim3(256), 0, st, (const T *)snap, CNT, flags);
             }
             hipLaunchKernelGGL(sweep_commit<T>, dim3((unsigned)cdiv(n, 256), nrhs), dim3(256), 0, st, n, (const T *)y,
-                               x, incx, ldx, (const int *)flags);
+                               x, incx, ldx, (const int *)flags, (int *)nullptr);
             cut_note(flags, st);
             cut.flags = flags;
             cut.g.p = 0;

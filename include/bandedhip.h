@@ -57,8 +57,8 @@ int bh_trim(void);
 /* What became of this thread's last factorisation or solve of the kind that can
  * run by blocks (gbtrf, pbtrf, sbldlt, each sweep of tbsv and of what is built
  * on it, gbtrs, gbtrs_part, gbtrs_blocked): *verdict_host is 1 when the blocks
- * agreed and are the result, 2 when the matrix was not tried (its sampled
- * diagonal does not dominate), 3 when they differed and the sequential kernels
+ * agreed and are the result, 2 when they were refused (the matrix's sampled
+ * columns do not dominate enough), 3 when they differed and the sequential kernels
  * ran, 0 when there were no blocks (or their memory has been given back).
  * *tries_host (may be NULL): how often blocks were launched.  Waits for that call. */
 int bh_cut_verdict(int *verdict_host, int *tries_host);
@@ -182,7 +182,9 @@ int bh_sgbtrs_blocked(bh_int n, bh_int kl, bh_int ku, bh_int nrhs, const float *
  * partitioned result's rounding error grows with the blocks' transfer
  * matrices; when an entry of one exceeds 1e8 (FP64) / 1e3 (FP32) in
  * magnitude the call runs bh_?gbtrs instead (B is written once, by whichever
- * ran).  One host synchronisation per call (that check).
+ * ran).  Factors whose diagonals dominate are solved by the blocks of bh_?gbtrs
+ * first, and have its bits then.  The host waits for these verdicts, not for
+ * the last kernel.
  * Same job as LAPACK.gbtrs! in ldiv!(::BandedLU, B) and
  * ldiv!(transpose(::BandedLU), B) (src/banded/linalg.jl:24-47). */
 int bh_gbtrs_part_workspace(char prec, bh_int n, bh_int kl, bh_int ku, bh_int nrhs, size_t *bytes);
