@@ -85,8 +85,8 @@ __device__ __forceinline__ bool cut_differ(float a, float b) {
 
 // One factorisation cut into blocks: block i factors columns start(i) ..
 // end(i)-1 and the rows they reach, in a copy of its own (ld = H = 2kl+ku+1),
-// as a system of its own.  g.p == 0: not cut (with flags: the sequential kernel
-// that runs only if the blocks failed).
+// as a system of its own.  g.p == 0: not cut (with flags: the sequential kernel,
+// launched behind the gate, which runs only if that is closed).
 template <typename T>
 struct LuCut {
     CutGeom g;
@@ -112,7 +112,8 @@ struct PbLane {
 // a wave to each, where they are longer than 64 entries: 42 -> 19 us at
 // 385 and 129 entries); closed when more than a quarter of them have num/4 times the sum of |a| off the
 // diagonal above |a_jj|.  One workgroup, so it writes both flags itself (and the
-// first one to a word of the host's, where there is one).
+// first one to a word of the host's, where there is one, and zeroes the caller's
+// two info words: a fill in front of the sequential kernel is a launch more).
 // rate > 0 (a symmetric matrix of which s1 holds one triangle): closed also
 // when the mean over the sampled columns of
 //     -sum over the stored entries at distance t of s^t a_t (z^t + z^-t) / a_jj,  z = 2^-rate,
@@ -127,6 +128,7 @@ struct PbLane {
 // times the other entries, simulated: what the test closes never agrees within
 // the lead-in; of what it leaves open, wide Laplacians at 1.25 to 3 times
 // dominance (kd = 64) do not agree either and pay for the trial.
+//
 // A set of entries of a column: rows r0 .. r0+h-1 of the band array, the
 // diagonal in row d (with `unit` it counts as 1); h = 0: no second set.
 struct CutSet {
@@ -134,9 +136,9 @@ struct CutSet {
 };
 template <typename T>
 __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld, int n, CutSet s1, CutSet s2, int num,
-                                                 float rate, int *flags, int *host) {
+                                                 float rate, int *flags, int *host, i64 *info) {
     __shared__ int weak[2];
-    __shared__ float part[2][64];
+    __shared__ float part[2][16];
     if (threadIdx.x < 2) weak[threadIdx.x] = 0;
     __syncthreads();
     const int lanes = s1.h > 64 ? 64 : 16, cols = 1024 / lanes, samples = 4 * cols;
@@ -148,43 +150,52 @@ __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld
         for (int off = lanes / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
         return T(4) * (s.unit ? T(1) : dabs(col[s.d])) >= T(num) * t;
     };
+    // per lane, over its entries of all its columns
     float mean[2] = {0.0f, 0.0f};
-    auto coherent = [&](const T *col, i64 c) {  // slots outside the matrix hold anything
-        T even = T(0), odd = T(0);
-        for (int r = q; r < s1.h; r += lanes) {
-            const int dist = s1.r0 + r - s1.d;
-            if (dist == 0 || c + dist < 0 || c + dist >= n) continue;
-            const float z = exp2f(rate * (float)dist);
-            const T t = col[s1.r0 + r] * T(z + 1.0f / z);
-            (dist & 1 ? odd : even) += t;
-        }
-        for (int off = lanes / 2; off > 0; off >>= 1) {
-            even += __shfl_xor(even, off, 64);
-            odd += __shfl_xor(odd, off, 64);
-        }
-        mean[0] -= (float)((even + odd) / col[s1.d]);
-        mean[1] -= (float)((even - odd) / col[s1.d]);
+    auto coherent = [&](const T *col, i64 c, int r, T w) {  // slots outside the matrix hold anything
+        const int dist = s1.r0 + r - s1.d;
+        if (dist == 0 || c + dist < 0 || c + dist >= n) return;
+        const float t = (float)(col[s1.r0 + r] * w / col[s1.d]);
+        mean[0] -= t;
+        mean[1] -= dist & 1 ? -t : t;
     };
+    const T *col[4];
+    i64 cs[4];
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
         // the golden section spreads the samples evenly without a stride, which a
         // grid's rows could be in step with
-        const i64 c = (i64)(((unsigned long long)((unsigned)(cols * it + g + 1) * 2654435769u) * (unsigned)n) >> 32);
-        const T *col = a + c * ld;
-        m1 += !strong(col, s1);
-        if (s2.h) m2 += !strong(col, s2);
-        if (rate > 0.0f) coherent(col, c);
+        cs[it] = (i64)(((unsigned long long)((unsigned)(cols * it + g + 1) * 2654435769u) * (unsigned)n) >> 32);
+        col[it] = a + cs[it] * ld;
+    }
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        m1 += !strong(col[it], s1);
+        if (s2.h) m2 += !strong(col[it], s2);
+    }
+    if (rate > 0.0f)
+        for (int r = q; r < s1.h; r += lanes) {
+            const float z = exp2f(rate * (float)(s1.r0 + r - s1.d));
+            const T w = T(z + 1.0f / z);
+#pragma unroll
+            for (int it = 0; it < 4; ++it) coherent(col[it], cs[it], r, w);
+        }
+    for (int off = 32; off > 0; off >>= 1) {
+        mean[0] += __shfl_xor(mean[0], off, 64);
+        mean[1] += __shfl_xor(mean[1], off, 64);
     }
     if (q == 0) {
         atomicAdd(&weak[0], m1);
         atomicAdd(&weak[1], m2);
-        part[0][g] = mean[0];
-        part[1][g] = mean[1];
+    }
+    if ((threadIdx.x & 63) == 0) {
+        part[0][threadIdx.x >> 6] = mean[0];
+        part[1][threadIdx.x >> 6] = mean[1];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         float t0 = 0.0f, t1 = 0.0f;
-        for (int i = 0; i < cols; ++i) {
+        for (int i = 0; i < 16; ++i) {
             t0 += part[0][i];
             t1 += part[1][i];
         }
@@ -192,6 +203,7 @@ __global__ void __launch_bounds__(1024) cut_gate(const T *__restrict__ a, i64 ld
             weak[0] > samples / 4 || weak[1] > samples / 4 || !(t0 <= (float)samples) || !(t1 <= (float)samples);
         flags[0] = closed;
         flags[1] = 0;
+        if (info) info[0] = info[1] = 0;
         cut_tell(host, closed);
     }
 }

@@ -209,8 +209,11 @@ __global__ void __launch_bounds__(256) lu_cut_check(LuCut<T> cut, int kv, int cm
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) lu_cut_commit(LuCut<T> cut, T *__restrict__ ab, i64 ld, i64 *__restrict__ ipiv) {
-    if (cut_failed(cut.flags)) return;
+__global__ void __launch_bounds__(256) lu_cut_commit(LuCut<T> cut, T *__restrict__ ab, i64 ld, i64 *__restrict__ ipiv,
+                                                     int *host) {
+    const bool failed = cut_failed(cut.flags);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) cut_tell(host, failed);
+    if (failed) return;
     const int blk = blockIdx.y, H = cut.H, s0 = cut.g.start(blk), c0 = cut.g.own(blk), nc = cut.g.end(blk) - c0;
     const T *src = cut.block_ab(blk) + (i64)(c0 - s0) * H;
     for (int e = blockIdx.x * 256 + threadIdx.x; e < nc * H; e += gridDim.x * 256) {
@@ -248,10 +251,11 @@ static CutGeom lu_cut_geom(i64 n, i64 kl, i64 ku, i64 blocks, int tries) {
 // its bits to agree, so it would only pay.  Measured, whole gbtrf call against the
 // sequential kernels: FP64 (8,8) n = 65536 0.40 ms against 31.3, (16,16)
 // n = 262144 1.7 against 125, (128,128) n = 65536 3.5 against 57.6 (FP32 2.0
-// against 37); what bounds it is the L + W steps of one block.  *ws: the blocks' memory with their
-// verdict in seq->flags, for the sequential kernel launched next (which does
-// nothing where the blocks succeeded) and to be freed after it; nullptr when
-// no blocks ran.
+// against 37); what bounds it is the L + W steps of one block.  The host learns
+// the gate's word while the sequential kernel, launched behind it, begins (or
+// finds the gate open and ends): a matrix that is not dominant pays the gate, not
+// the blocks' launches too.  kCutDone: the factors and pivots are in place,
+// info 0; kCutLaunched: the sequential kernel runs already; kCutNot: neither.
 int blk_shape_for(i64 kl, i64 ku);
 size_t mfma_lds_bytes(i64 kl, i64 elem);
 
@@ -268,55 +272,64 @@ static int lu_kernel_launch(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 lda
     }
 }
 
+enum CutOutcome { kCutNot, kCutLaunched, kCutDone };
+
 template <typename T>
-static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, void **ws_out, LuCut<T> *seq) {
-    *ws_out = nullptr;
+static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, CutOutcome *out) {
+    *out = kCutNot;
     if (kl < 1 || !cut_enabled()) return BH_OK;
     hipStream_t st = stream();
     const int kv = (int)(kl + ku), H = (int)(2 * kl + ku + 1);
     // one workgroup per CU for the MFMA and the blocked kernel (their LDS), one wave per SIMD for the lane kernel
     const i64 blocks = kind == kLuLane ? 1024 : 256;
+    struct Free {
+        void *p = nullptr;
+        hipStream_t st;
+        ~Free() { cut_free(p, st); }
+    };
     for (int tries = 0; tries < 2; ++tries) {
         const CutGeom g = lu_cut_geom<T>(n, kl, ku, blocks, tries);
-        if (g.p == 0) return BH_OK;
+        int *host = g.p > 0 ? cut_host_words() : nullptr;
+        if (!host) return BH_OK;
         const size_t ba = (((size_t)g.p * g.span() * H * sizeof(T)) + 255) & ~(size_t)255;
         const size_t bp = (size_t)g.p * g.span() * sizeof(i64), bi = (size_t)g.p * 2 * sizeof(i64);
-        char *ws = (char *)cut_alloc(ba + bp + bi + 256, st);
+        Free mem;
+        mem.st = st;
+        char *ws = (char *)(mem.p = cut_alloc(ba + bp + bi + 256, st));
         if (!ws) return BH_OK;
         int *flags = (int *)(ws + ba + bp + bi);
         const LuCut<T> cut{g, flags, (T *)ws, (i64 *)(ws + ba), (i64 *)(ws + ba + bp), H, (int)kl};
         hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                           CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, 0.0f, flags, (int *)nullptr);
+                           CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, 0.0f, flags, host, dinfo);
+        BH_LAUNCH_CHECK();
+        cut_note(flags, st);
+        int r = -1;
+        if (tries == 0) {
+            LuCut<T> seq{};
+            seq.flags = flags;
+            r = lu_kernel_launch<T>(kind, n, kl, ku, ab, ldab, ipiv, dinfo, st, &seq);
+        }
+        const int closed = cut_poll(host, st);
+        if (r != BH_OK && r != -1) return r;  // -1: not the whole system (its 32-bit offsets), its blocks perhaps
+        if (closed < 0) BH_HIP(hipStreamSynchronize(st));
+        if (closed != 0) {
+            *out = r == BH_OK ? kCutLaunched : kCutNot;
+            return BH_OK;
+        }
         const unsigned gx = (unsigned)imin(64, cdiv((i64)g.span() * H, 1024));
         hipLaunchKernelGGL(lu_cut_copy<T>, dim3(gx, g.p), dim3(256), 0, st, cut, (const T *)ab, ldab, kv);
-        const int r = lu_kernel_launch<T>(kind, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);
-        if (r != BH_OK) {
-            cut_free(ws, st);
-            return r == -1 ? BH_OK : r;  // -1: the kernel does not take this band
-        }
-        cut_note(flags, st);
+        r = lu_kernel_launch<T>(kind, n, kl, ku, cut.ab, H, cut.ipiv, cut.info, st, &cut);
+        if (r != BH_OK) return r == -1 ? BH_OK : r;  // -1: the kernel does not take this band
         hipLaunchKernelGGL(lu_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, kv, (int)up16(kv), flags);
-        hipLaunchKernelGGL(lu_cut_commit<T>, dim3(gx, g.p), dim3(256), 0, st, cut, ab, ldab, ipiv);
-        hipError_t e = hipGetLastError();
-        // Long enough that four times the lead-in is still little of the
-        // chain: look at the verdict here (one wait) and try once more.
-        int fl[2] = {0, 0};
-        if (tries == 0 && n >= 32 * (i64)(g.L + 4 * g.W)) {
-            if (e == hipSuccess) e = hipMemcpyAsync(fl, flags, sizeof fl, hipMemcpyDeviceToHost, st);
-            if (e == hipSuccess) e = hipStreamSynchronize(st);
+        hipLaunchKernelGGL(lu_cut_commit<T>, dim3(gx, g.p), dim3(256), 0, st, cut, ab, ldab, ipiv, host + 1);
+        BH_LAUNCH_CHECK();
+        BH_HIP(hipStreamSynchronize(st));
+        if (host[1] == 0) {
+            *out = kCutDone;
+            return BH_OK;
         }
-        if (e != hipSuccess) {
-            cut_free(ws, st);
-            return hip_fail(e, "gbtrf (cut)", __FILE__, __LINE__);
-        }
-        if (fl[0] == 0 && fl[1] != 0) {
-            cut_free(ws, st);
-            continue;
-        }
-        *seq = LuCut<T>{};
-        seq->flags = flags;
-        *ws_out = ws;
-        return BH_OK;
+        // long enough that four times the lead-in is still little of the chain: once more
+        if (n < 32 * (i64)(g.L + 4 * g.W)) return BH_OK;
     }
     return BH_OK;
 }
@@ -349,36 +362,24 @@ static int gbtrf_impl(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
         kind = kLuLane;
     else if (ov == 0 && kl >= 16 && blk_shape_for(kl, ku) >= 0)
         kind = kLuBlk;
-    void *ws = nullptr;
-    LuCut<T> seq{};
+    CutOutcome cut = kCutNot;
     cut_begin();
     if (m == n && kind != kLuNone) {
-        const int cs = gbtrf_cut<T>(kind, n, kl, ku, ab, ldab, ipiv, &ws, &seq);
+        const int cs = gbtrf_cut<T>(kind, n, kl, ku, ab, ldab, ipiv, dinfo, &cut);
         if (cs) return cs;
+        if (cut == kCutDone) return BH_OK;
     }
-    struct Free {
-        void *p;
-        ~Free() { cut_free(p, stream()); }
-    } free_ws{ws};
-    BH_HIP(hipMemsetAsync(dinfo, 0, 2 * sizeof(i64), stream()));
+    if (cut == kCutNot) BH_HIP(hipMemsetAsync(dinfo, 0, 2 * sizeof(i64), stream()));
     // The MFMA-blocked factorisation (pivots equal xGBTF2's, factors to
     // rounding): where the reference itself runs blocked xGBTRF (ku >= 65,
     // kl >= 32), and for long systems with kl, ku >= 8, where the one-wave
     // chain of the narrow kernels is the longer path (n = 262144, (16,16):
     // 142 ms against 278 ms).  Shorter narrow systems keep the bit-exact
     // xGBTF2 kernels.
-    if (mfma)
-        st = mfma_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), ws ? &seq : nullptr);
-    else if (ws)
-        st = lu_kernel_launch<T>(kind, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), &seq);
-    if (st == -1 && ws) {
-        // the blocks' kernel does not take the whole system (its 32-bit
-        // offsets): only their verdict tells whether another one has to run
-        int fl[2];
-        BH_HIP(hipMemcpyAsync(fl, seq.flags, sizeof fl, hipMemcpyDeviceToHost, stream()));
-        BH_HIP(hipStreamSynchronize(stream()));
-        if (fl[0] == 0 && fl[1] == 0) return BH_OK;
-    }
+    if (cut == kCutLaunched)
+        st = BH_OK;
+    else if (mfma)
+        st = mfma_gbtrf_launch<T>(m, n, kl, ku, ab, ldab, ipiv, dinfo, stream(), nullptr);
     // The one-wave lane kernel exists for kl <= 16; above 16 the
     // blocked kernel beats the generic one-wave kernel (at n = 65536, (24,24):
     // 113.5 ms against 278.6 ms, identical factors), so it goes first there.

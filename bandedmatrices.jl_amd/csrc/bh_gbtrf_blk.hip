@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(64 * (NW + 1)) gbtrf_blk_kernel(BlkArgs<T> s) 
         s.ipiv = s.cut.ipiv + (i64)blk * s.cut.g.span();
         s.info = s.cut.info + 2 * blk;
     } else if (s.cut.flags && !cut_failed(s.cut.flags)) {
-        return;  // the blocks of a cut system have done it
+        return;  // the gate is open: the blocks of a cut system do it
     }
     const int m = s.m, n = s.n, kl = s.kl, ku = s.ku, kv = kl + ku, H = kv + 1;
     const i64 ld = s.ldab;

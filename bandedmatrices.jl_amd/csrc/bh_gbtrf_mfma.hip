@@ -284,7 +284,7 @@ __global__ void __launch_bounds__(64 * QWAVES) gbtrf_mfma_kernel(QArgs<T> s) {
         s.ipiv = s.cut.ipiv + (i64)blk * s.cut.g.span();
         s.info = s.cut.info + 2 * blk;
     } else if (s.cut.flags && !cut_failed(s.cut.flags)) {
-        return;  // the blocks of a cut system have done it
+        return;  // the gate is open: the blocks of a cut system do it
     }
     const int m = s.m, n = s.n, kl = s.kl, ku = s.ku, kv = kl + ku;
     const int R = s.R, RT = s.RT, RP = s.RP;
@@ -802,7 +802,7 @@ size_t mfma_lds_bytes(i64 kl, i64 elem) {
 // static words (under 4 KiB), within 160 KiB).
 // With a cut it runs the blocks of a cut system in their own copies, whose
 // fill-in rows are already zero (ab, ipiv and dinfo are not read); with
-// cut->g.p == 0 it does nothing unless cut->flags say that the blocks failed.
+// cut->g.p == 0 it does nothing unless cut->flags say that the gate is closed.
 template <typename T>
 int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<T> *cut) {

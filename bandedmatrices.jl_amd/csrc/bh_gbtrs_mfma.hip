@@ -708,7 +708,7 @@ int trs_blocked_solve(i64 n, i64 kl, i64 ku, i64 nrhs, const T *ab, i64 ldab, co
             int *flags = (int *)(ws + 2 * by + sl + su);
             const int kd = (int)(kl + ku);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, ab, ldab, (int)n, CutSet{0, kd + 1, kd, 0},
-                               CutSet{kd, (int)kl + 1, kd, 1}, 5, 0.0f, flags, (int *)nullptr);
+                               CutSet{kd, (int)kl + 1, kd, 1}, 5, 0.0f, flags, (int *)nullptr, (i64 *)nullptr);
             hipLaunchKernelGGL(kf, dim3(grid.x, gl.p), block, fl, st, (const T *)B, ldb, Y, n, (int)nrhs, L, idx, rec,
                                SweepCut<T>{gl, flags, snl});
             hipLaunchKernelGGL(sweep_check<T>, dim3(gl.p - 1, grid.x), dim3(256), 0, st, (const T *)snl, cl, flags);

@@ -442,7 +442,7 @@ int ring_run(K kern, bool trans, int how, i64 n, i64 kl, i64 ku, i64 nrhs, const
             flags = (int *)(ws + 2 * by + su + sl);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, ab, ld, (int)n,
                                CutSet{0, (int)kd + 1, (int)kd, 0}, CutSet{(int)kd, kl ? (int)kl + 1 : 0, (int)kd, 1},
-                               5, 0.0f, flags, host);
+                               5, 0.0f, flags, host, (i64 *)nullptr);
             cut_note(flags, st);
         }
     }

@@ -31,7 +31,7 @@ struct BatchDesc {
 
 // Single-system gbtrf through the rotating-register kernel (kl <= 16, kl + ku <= 63, band storage under 2 GiB), or -1.  With a cut it
 // runs the blocks of a cut system, one wave each; with cut->g.p == 0 it does
-// nothing unless cut->flags say that the blocks failed.
+// nothing unless cut->flags say that the gate is closed.
 int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, double *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<double> *cut);
 int lane_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, float *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(64) gbtrf_lane_kernel(int m, int n, int ku, T 
         ipiv = cut.ipiv + (i64)blk * cut.g.span();
         info = cut.info + 2 * blk;
     } else if (cut.flags && !cut_failed(cut.flags)) {
-        return;  // the blocks of a cut system have done it
+        return;  // the gate is open: the blocks of a cut system do it
     }
     const int r = lane_gbsv_wave<T, KL, false, 16>(m, n, ku, ab, ld, ipiv, nullptr);
     if (threadIdx.x == 0) *info = r;

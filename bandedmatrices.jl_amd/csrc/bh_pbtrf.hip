@@ -42,7 +42,8 @@ namespace bh {
 template <typename T>
 PbLane pbtrf_lane_geom(i64 n, i64 kd, i64 ldab);
 template <typename T>
-int pbtrf_lane_run(const PbLane &g, i64 n, i64 kd, T *ab, i64 ldab, T *out, T *seam, int *flags, hipStream_t st);
+int pbtrf_lane_run(const PbLane &g, i64 n, i64 kd, T *ab, i64 ldab, T *out, T *seam, int *flags, int *host,
+                   hipStream_t st);
 
 namespace {
 
@@ -55,8 +56,8 @@ __device__ __forceinline__ float dsqrt<float>(float x) { return __builtin_sqrtf(
 
 constexpr int kPbRegs = 24;  // staged values per thread: chunk columns x (kd+1) <= kPbRegs x threads
 
-// One factorisation by blocks; g.p == 0: the whole of it (with flags: only if
-// the blocks failed).
+// One factorisation by blocks; g.p == 0: the whole of it (with flags: only
+// behind a closed gate).
 template <typename T>
 struct PbCut {
     CutGeom g;
@@ -225,8 +226,10 @@ __global__ void __launch_bounds__(256) pb_cut_check(PbCut<T> cut, int kd, int up
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) pb_cut_commit(PbCut<T> cut, int kd, T *__restrict__ ab, i64 ldab) {
-    if (cut_failed(cut.flags)) return;
+__global__ void __launch_bounds__(256) pb_cut_commit(PbCut<T> cut, int kd, T *__restrict__ ab, i64 ldab, int *host) {
+    const bool failed = cut_failed(cut.flags);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) cut_tell(host, failed);
+    if (failed) return;
     const int blk = blockIdx.y, H = kd + 1, c0 = cut.g.own(blk), nc = cut.g.end(blk) - c0;
     const T *src = cut.block(blk, kd) + (i64)(c0 - cut.g.start(blk)) * H;
     for (int e = blockIdx.x * 256 + threadIdx.x; e < nc * H; e += gridDim.x * 256) {
@@ -284,8 +287,10 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
     hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // By blocks where |a_jj| is at least 1.75 times the sum of its stored
     // row or column (half of the off-diagonal entries: plain dominance is 2
-    // on average) and the gate's rate test leaves room for the lead-in; behind
-    // them the whole chain, which does nothing where the blocks agreed.
+    // on average) and the gate's rate test leaves room for the lead-in.  The
+    // whole chain is launched behind the gate, ends at once where that is open, and
+    // the host learns the gate's word meanwhile: then the blocks, and the chain
+    // again where they differed.
     PbCut<T> cut{};
     char *ws = nullptr;
     cut_begin();
@@ -293,50 +298,55 @@ int pbtrf_impl(char uplo, i64 n, i64 kd, T *ab, i64 ldab, i64 *info_host) {
     // an upper Cholesky with kd <= 8: one lane per block (0.32 ms with a
     // workgroup per block at n = 65536, kd = 8, FP64; 0.13 with a lane)
     const PbLane gl = up && !LDL ? pbtrf_lane_geom<T>(n, kd, ldab) : PbLane{0, 0, 0};
-    if (e == hipSuccess && gl.p > 0 && cut_enabled()) {
-        const size_t bo = ((size_t)n * H * sizeof(T) + 255) & ~(size_t)255;
-        const size_t bs = ((size_t)2 * kd * H * gl.p * sizeof(T) + 255) & ~(size_t)255;
-        ws = (char *)cut_alloc(bo + bs + 256, st);
-        if (ws) {
-            int *flags = (int *)(ws + bo + bs);
-            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, (int)kd, 0}, CutSet{}, 7, cut_rate<T>(gl.W), flags,
-                               (int *)nullptr);
-            const int r = pbtrf_lane_run<T>(gl, n, kd, ab, ldab, (T *)ws, (T *)(ws + bo), flags, st);
-            if (r != BH_OK) {
-                cut_free(ws, st);
-                return r;
-            }
-            cut_note(flags, st);
-            cut.flags = flags;
-            e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
-        }
-    } else if (e == hipSuccess && g.p > 0 && cut_enabled()) {
-        const size_t bo = ((size_t)g.p * (g.span() + kd) * H * sizeof(T) + 255) & ~(size_t)255;
-        const size_t bi = (size_t)g.p * sizeof(i64);
-        ws = (char *)cut_alloc(bo + bi + 256, st);
-        if (ws) {
-            int *flags = (int *)(ws + bo + bi);
-            cut = PbCut<T>{g, flags, (T *)ws, (i64 *)(ws + bo)};
-            hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
-                               CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, cut_rate<T>(g.W), flags,
-                               (int *)nullptr);
-            hipLaunchKernelGGL(kern, dim3(g.p), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, (T *)nullptr,
-                               (i64)0, (i64 *)nullptr, (int)B, cut);
-            hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, cut, (int)kd, (int)up, flags);
-            hipLaunchKernelGGL(pb_cut_commit<T>, dim3((unsigned)imin(16, cdiv(g.L * H, 256)), g.p), dim3(256), 0, st,
-                               cut, (int)kd, ab, ldab);
-            cut_note(flags, st);
-            e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
-            cut.g.p = 0;
-        }
-    }
-    if (e == hipSuccess) {
+    const bool lane = gl.p > 0;
+    const size_t bo = lane ? ((size_t)n * H * sizeof(T) + 255) & ~(size_t)255
+                           : ((size_t)g.p * (g.span() + kd) * H * sizeof(T) + 255) & ~(size_t)255;
+    const size_t bs = lane ? ((size_t)2 * kd * H * gl.p * sizeof(T) + 255) & ~(size_t)255 : (size_t)g.p * sizeof(i64);
+    int *host = e == hipSuccess && (lane || g.p > 0) && cut_enabled() ? cut_host_words() : nullptr;
+    if (host) ws = (char *)cut_alloc(bo + bs + 256, st);
+    struct Free {
+        void *p;
+        hipStream_t st;
+        ~Free() { cut_free(p, st); }
+    } free_ws{ws, st};
+    if (e == hipSuccess && !ws) e = hipMemsetAsync(dinfo, 0, sizeof(i64), st);
+    auto chain = [&] {  // cut.g.p == 0: whole, with flags only behind a closed gate
         hipLaunchKernelGGL(kern, dim3(1), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, ab, ldab, dinfo,
                            (int)B, cut);
-        e = hipGetLastError();
+        return hipGetLastError();
+    };
+    bool run = true;  // the chain is still to be launched
+    if (e == hipSuccess && ws) {
+        int *flags = (int *)(ws + bo + bs);
+        hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, (const T *)ab, ldab, (int)n,
+                           CutSet{0, (int)H, up ? (int)kd : 0, 0}, CutSet{}, 7, cut_rate<T>(lane ? gl.W : g.W), flags,
+                           host, dinfo);
+        BH_LAUNCH_CHECK();
+        cut_note(flags, st);
+        cut.flags = flags;
+        e = chain();
+        cut.flags = nullptr;
+        const int closed = cut_poll(host, st);
+        if (e == hipSuccess && closed < 0) e = hipStreamSynchronize(st);
+        run = closed == 0;
+        if (e == hipSuccess && closed == 0) {
+            if (lane) {
+                const int r = pbtrf_lane_run<T>(gl, n, kd, ab, ldab, (T *)ws, (T *)(ws + bo), flags, host + 1, st);
+                if (r != BH_OK) return r;
+            } else {
+                const PbCut<T> blk{g, flags, (T *)ws, (i64 *)(ws + bo)};
+                hipLaunchKernelGGL(kern, dim3(g.p), dim3(nt), lds, st, (int)n, (int)kd, (const T *)ab, ldab, (T *)nullptr,
+                                   (i64)0, (i64 *)nullptr, (int)B, blk);
+                hipLaunchKernelGGL(pb_cut_check<T>, dim3(g.p), dim3(256), 0, st, blk, (int)kd, (int)up, flags);
+                hipLaunchKernelGGL(pb_cut_commit<T>, dim3((unsigned)imin(16, cdiv(g.L * H, 256)), g.p), dim3(256), 0, st,
+                                   blk, (int)kd, ab, ldab, host + 1);
+            }
+            e = hipGetLastError();
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            if (e == hipSuccess && host[1] == 0) return BH_OK;  // *info_host is 0
+        }
     }
-    cut_free(ws, st);
+    if (e == hipSuccess && run) e = chain();
     if (e == hipSuccess) e = hipMemcpyAsync(info_host, dinfo, sizeof(i64), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(e, "pbtrf", __FILE__, __LINE__);

@@ -156,8 +156,10 @@ __global__ void __launch_bounds__(256) pbtrf_lane_check(int p, int cnt, const T 
 
 template <typename T>
 __global__ void __launch_bounds__(256) pbtrf_lane_commit(int n, int H, const T *__restrict__ out, T *__restrict__ ab, i64 lda,
-                                                         const int *flags) {
-    if (cut_failed(flags)) return;
+                                                         const int *flags, int *host) {
+    const bool failed = cut_failed(flags);
+    if (blockIdx.x == 0 && threadIdx.x == 0) cut_tell(host, failed);
+    if (failed) return;
     const i64 e = (i64)blockIdx.x * 256 + threadIdx.x;
     if (e >= (i64)n * H) return;
     const i64 c = e / H;
@@ -185,7 +187,8 @@ PbLane pbtrf_lane_geom(i64 n, i64 kd, i64 ldab) {
 
 // out: n x (kd+1), seam: 2 kd (kd+1) p entries.
 template <typename T>
-int pbtrf_lane_run(const PbLane &g, i64 n, i64 kd, T *ab, i64 ldab, T *out, T *seam, int *flags, hipStream_t st) {
+int pbtrf_lane_run(const PbLane &g, i64 n, i64 kd, T *ab, i64 ldab, T *out, T *seam, int *flags, int *host,
+                   hipStream_t st) {
     const dim3 grid((unsigned)cdiv(g.p, 64));
     switch ((int)kd) {
 #define BH_PL_CASE(Kv)                                                                                              \
@@ -202,13 +205,15 @@ int pbtrf_lane_run(const PbLane &g, i64 n, i64 kd, T *ab, i64 ldab, T *out, T *s
     hipLaunchKernelGGL(pbtrf_lane_check<T>, dim3((unsigned)cdiv(g.p, 256), imin(cnt, 16)), dim3(256), 0, st, g.p, cnt,
                        (const T *)seam, flags);
     hipLaunchKernelGGL(pbtrf_lane_commit<T>, dim3((unsigned)cdiv(n * (kd + 1), 256)), dim3(256), 0, st, (int)n,
-                       (int)kd + 1, (const T *)out, ab, ldab, (const int *)flags);
+                       (int)kd + 1, (const T *)out, ab, ldab, (const int *)flags, host);
     return BH_OK;
 }
 
 template PbLane pbtrf_lane_geom<double>(i64, i64, i64);
 template PbLane pbtrf_lane_geom<float>(i64, i64, i64);
-template int pbtrf_lane_run<double>(const PbLane &, i64, i64, double *, i64, double *, double *, int *, hipStream_t);
-template int pbtrf_lane_run<float>(const PbLane &, i64, i64, float *, i64, float *, float *, int *, hipStream_t);
+template int pbtrf_lane_run<double>(const PbLane &, i64, i64, double *, i64, double *, double *, int *, int *,
+                                    hipStream_t);
+template int pbtrf_lane_run<float>(const PbLane &, i64, i64, float *, i64, float *, float *, int *, int *,
+                                   hipStream_t);
 
 }  // namespace bh

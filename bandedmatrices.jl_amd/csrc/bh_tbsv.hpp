@@ -263,7 +263,7 @@ int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx,
             int *flags = (int *)(ws + by + bs);
             T *y = (T *)ws, *snap = (T *)(ws + by);
             hipLaunchKernelGGL(cut_gate<T>, dim3(1), dim3(1024), 0, st, a, lda, n,
-                               CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, 0.0f, flags, (int *)nullptr);
+                               CutSet{0, k + 1, TbMode<MODE>::UPPER ? k : 0, (int)unit}, CutSet{}, 5, 0.0f, flags, (int *)nullptr, (i64 *)nullptr);
             if (gl.p > 0) {
                 const int r = tbsv_lane_run(gl, TbMode<MODE>::ASC, n, k, a, lda, x, incx, ldx, nrhs, unit, y, snap,
                                             flags, st);
