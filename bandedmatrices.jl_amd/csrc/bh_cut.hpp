@@ -14,8 +14,11 @@
 // for the same steps before its own began.  The first block starts where the
 // chain starts, so equality at every seam makes every block's result the
 // sequential chain's, bit for bit.  If a seam differs nothing has been
-// written to the caller's arrays yet and the sequential kernel, launched
-// behind the blocks with the verdict as its condition, does the work.
+// written to the caller's arrays yet and the sequential kernel does the work:
+// launched behind the blocks with the verdict as its condition where the call
+// waits for nothing (tbsv, gbtrs, gbtrs_blocked: a refused matrix pays 11-25 us
+// of gate and empty launches), by the host, which learns the verdicts on the
+// way, where it waits anyway (gbtrf, pbtrf, gbtrs_part: 15-20 us).
 //
 // The check decides the result; the gate only decides whether trying is worth
 // its time (it samples columns for diagonal dominance: without it a matrix
@@ -262,9 +265,12 @@ __global__ void __launch_bounds__(256) sweep_commit(int n, const T *__restrict__
 }
 
 // Groups of a sweep over n steps with bandwidth k, nrhs vectors.  Lead-in:
-// measured on the factors of dominant matrices (k = 2 .. 64) the windows
-// agree after 13-23 k steps in FP64 and 7-10 k in FP32; two groups more cover
-// the window itself.  Own groups: about 2048 waves (two per SIMD) over all
+// measured on the factors of dominant random matrices the windows agree after
+// 12-18 k steps in FP64 (k = 4 .. 64; 23 k at k = 2) and 7-10 k in FP32; 20 k
+// and 10 k, with nw whole groups more for the window itself (64 steps and up,
+// which at k = 2 is another 32 k).  Factors of constant sparse bands forget more
+// slowly (a five-point operator at 1.25 to 1.5 times dominance: 28-41 k): those
+// differ and pay for the trial.  Own groups: about 2048 waves (two per SIMD) over all
 // vectors, and not under half the lead-in, which every block repeats.
 template <typename T>
 inline CutGeom sweep_geom(i64 n, i64 k, i64 nrhs, i64 nw) {

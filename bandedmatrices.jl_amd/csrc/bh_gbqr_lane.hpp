@@ -1,4 +1,4 @@
-// bh_gbqr_lane.hpp -- banded Householder QR of narrow bands (l <= 8) and the
+// bh_gbqr_lane.hpp -- banded Householder QR of narrow bands (l <= 7) and the
 // application of its Q', one wave, the band's subdiagonal count fixed at
 // compile time.  Instantiated per element type in bh_gbqr_lane_{d,s}.hip
 // (BH_QL_T); bh_gbqr.hip calls the launchers.

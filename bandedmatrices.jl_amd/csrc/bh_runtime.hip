@@ -210,7 +210,8 @@ bool cut_enabled() {
 int *cut_host_words() {
     if (!g_cut.host) {
         const RelaxedCapture relaxed;
-        if (hipHostMalloc((void **)&g_cut.host, kCutWords * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc((void **)&g_cut.host, kCutWords * sizeof(int),
+                          hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
             g_cut.host = nullptr;
             return nullptr;

@@ -13,14 +13,14 @@
 
 namespace bh {
 
-// The blocks of a 'N' solve (ASC: lower, else upper), their seam checks into
-// flags; y (n x nrhs) takes the result.  Workspace for the windows: lane_snap
-// bytes.  False: a k or size these do not take.
+// The blocks of a 'N' solve; p = 0: a k or size they do not take.
 struct TbsvLane {
     int p = 0, L = 0, W = 0;  // blocks, own steps, lead-in
 };
 TbsvLane tbsv_lane_geom(i64 n, i64 k, i64 lda, i64 incx, i64 ldx, i64 nrhs, int elem);
 inline size_t tbsv_lane_bytes(const TbsvLane &g, i64 k, i64 nrhs, size_t elem) { return (size_t)2 * g.p * k * nrhs * elem; }
+// Runs them (asc: lower, else upper) and their seam checks into flags; y (n x
+// nrhs) takes the result, snap (tbsv_lane_bytes) the windows.
 int tbsv_lane_run(const TbsvLane &g, bool asc, int n, int k, const double *a, i64 lda, const double *x, int incx, i64 ldx,
                   int nrhs, bool unit, double *y, double *snap, int *flags, hipStream_t st);
 int tbsv_lane_run(const TbsvLane &g, bool asc, int n, int k, const float *a, i64 lda, const float *x, int incx, i64 ldx,
