@@ -303,8 +303,10 @@ static int gbtrf_cut(LuKernel kind, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 
                            CutSet{(int)kl, (int)(kl + ku + 1), kv, 0}, CutSet{}, 5, 0.0f, flags, host, dinfo);
         BH_LAUNCH_CHECK();
         cut_note(flags, st);
+        // (the MFMA kernel's fill of whole columns takes some 30 us to find the
+        // gate open, n = 262144; its chains are long enough to wait for the word)
         int r = -1;
-        if (tries == 0) {
+        if (tries == 0 && kind != kLuMfma) {
             LuCut<T> seq{};
             seq.flags = flags;
             r = lu_kernel_launch<T>(kind, n, kl, ku, ab, ldab, ipiv, dinfo, st, &seq);

@@ -283,8 +283,6 @@ __global__ void __launch_bounds__(64 * QWAVES) gbtrf_mfma_kernel(QArgs<T> s) {
         s.n = s.cut.cols(blk);
         s.ipiv = s.cut.ipiv + (i64)blk * s.cut.g.span();
         s.info = s.cut.info + 2 * blk;
-    } else if (s.cut.flags && !cut_failed(s.cut.flags)) {
-        return;  // the gate is open: the blocks of a cut system do it
     }
     const int m = s.m, n = s.n, kl = s.kl, ku = s.ku, kv = kl + ku;
     const int R = s.R, RT = s.RT, RP = s.RP;
@@ -778,8 +776,7 @@ int mfma_launch_one(const QArgs<T> &a, hipStream_t st) {
 // step and those of column j+kv at step j (j < min(m,n)); zero them all up
 // front (rows whose row index is >= 0 only).
 template <typename T>
-__global__ void gbtrf_zero_fill(T *ab, i64 ld, int n, int mn, int kl, int ku, const int *flags) {
-    if (flags && !cut_failed(flags)) return;
+__global__ void gbtrf_zero_fill(T *ab, i64 ld, int n, int mn, int kl, int ku) {
     const int kv = kl + ku;
     const int c = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
     const int cend = qmin(n, mn + kv);
@@ -801,8 +798,7 @@ size_t mfma_lds_bytes(i64 kl, i64 elem) {
 // in at most four slots per lane and the LDS buffers, with the kernel's
 // static words (under 4 KiB), within 160 KiB).
 // With a cut it runs the blocks of a cut system in their own copies, whose
-// fill-in rows are already zero (ab, ipiv and dinfo are not read); with
-// cut->g.p == 0 it does nothing unless cut->flags say that the gate is closed.
+// fill-in rows are already zero (ab, ipiv and dinfo are not read).
 template <typename T>
 int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, i64 *dinfo, hipStream_t st,
                       const LuCut<T> *cut) {
@@ -818,7 +814,7 @@ int mfma_gbtrf_launch(i64 m, i64 n, i64 kl, i64 ku, T *ab, i64 ldab, i64 *ipiv, 
     if (a.cut.g.p == 0 && cend > ku + 1) {
         const int per = 4;  // columns per 256-thread block
         hipLaunchKernelGGL(gbtrf_zero_fill<T>, dim3((cend + per - 1) / per), dim3(64 * per), 0, st, ab, ldab, (int)n,
-                           mn, (int)kl, (int)ku, a.cut.flags);
+                           mn, (int)kl, (int)ku);
         BH_LAUNCH_CHECK();
     }
     const int PR = (R + 63) / 64;
