@@ -249,8 +249,8 @@ static CutGeom lu_cut_geom(i64 n, i64 kl, i64 ku, i64 blocks, int tries) {
 // 1.25 times the rest of their column: the measured families are at 2 and
 // more, and a matrix near 1 (the second difference) forgets too slowly for
 // its bits to agree, so it would only pay.  Measured, whole gbtrf call against the
-// sequential kernels: FP64 (8,8) n = 65536 0.40 ms against 31.3, (16,16)
-// n = 262144 1.7 against 125, (128,128) n = 65536 3.5 against 57.6 (FP32 2.0
+// sequential kernels: FP64 (8,8) n = 10000 0.17 ms against 5.3, (16,16)
+// n = 262144 0.75 against 125, (128,128) n = 65536 2.7 against 57.6 (FP32 1.29
 // against 37); what bounds it is the L + W steps of one block.  The host learns
 // the gate's word while the sequential kernel, launched behind it, begins (or
 // finds the gate open and ends): a matrix that is not dominant pays the gate, not

@@ -242,8 +242,9 @@ __global__ void __launch_bounds__(256) pb_cut_commit(PbCut<T> cut, int kd, T *__
 // kd+1 .. kd+2 under entries U(-1,1) (kd = 2 .. 64): the bits agree after
 // 8-12 kd columns in FP64 and 4-6 kd in FP32; four blocks to a CU (small
 // windows: their barriers overlap), not under half the lead-in each.  Factor
-// and solve at n = 65536, kd = 8, FP64: 73.7 -> 0.71 ms; the chain of one
-// block (L + W steps of 1.1 us) bounds it.
+// and solve at n = 65536, kd = 8, FP64: 73.7 -> 0.71 ms (0.49 with the upper
+// factor by lanes, bh_pbtrf_lane.hip); the chain of one block (L + W steps of
+// 1.1 us) bounds it.
 template <typename T>
 CutGeom pb_cut_geom(i64 n, i64 kd) {
     const i64 W = (sizeof(T) == 8 ? 14 : 8) * kd + 32;

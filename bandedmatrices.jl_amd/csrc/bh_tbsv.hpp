@@ -239,9 +239,9 @@ __global__ void __launch_bounds__(kTbBlock) tbsv_block(int n, int k, const T *__
 // The ring solve: by blocks where the triangle's columns are dominated by
 // their diagonal (1.25 times the rest, or 1 for a unit diagonal), and behind
 // them the whole sweep, which does nothing where the blocks agreed.  Measured
-// 'N' upper FP64: n = 2^20, k = 8 143 -> 0.31 ms by rings, 0.156 by lanes (rings: 0.3 us a step
+// 'N' upper FP64: n = 2^20, k = 8 143 -> 0.31 ms by rings, 0.11 by lanes (rings: 0.3 us a step
 // over a block's steps with two waves to a SIMD); a triangle that fails the gate pays the gate
-// and four empty launches, about 25 us.
+// and three empty launches, 11 us.
 template <typename T, int MODE, int NW, int PFD>
 int tbsv_ring_launch(int n, int k, const T *a, i64 lda, T *x, int incx, i64 ldx, int nrhs, bool unit, hipStream_t st) {
     constexpr int CNT = 64 * NW;
