@@ -270,25 +270,26 @@ void *cut_alloc(size_t bytes, hipStream_t st) {
         if (!c) return nullptr;
         c->busy = true;
     }
-    const RelaxedCapture relaxed;
     bool ok = true;
-    if (c->p && (c->dev != dev || c->bytes < bytes))
-        ok = cut_release(*c);
-    else if (c->p)
+    if (c->p && c->dev == dev && c->bytes >= bytes) {
         // also on what looks like the same stream: it may be a new one at the
         // handle of a destroyed one whose work still runs
         ok = hipStreamWaitEvent(st, c->done, 0) == hipSuccess;
-    if (ok && c->done && c->dev != dev) {
-        (void)hipEventDestroy(c->done);
-        c->done = nullptr;
-    }
-    if (ok && !c->done) ok = hipEventCreateWithFlags(&c->done, hipEventDisableTiming) == hipSuccess;
-    if (ok && !c->p) {
-        // some room to grow, within what is kept
-        const size_t nb = bytes > kCutKeep ? bytes : (bytes + bytes / 4 < kCutKeep ? bytes + bytes / 4 : kCutKeep);
-        ok = device_alloc(&c->p, nb) == hipSuccess;
-        c->bytes = ok ? nb : 0;
-        if (!ok) c->p = nullptr;
+    } else {
+        const RelaxedCapture relaxed;
+        ok = cut_release(*c);
+        if (ok && c->done && c->dev != dev) {
+            (void)hipEventDestroy(c->done);
+            c->done = nullptr;
+        }
+        if (ok && !c->done) ok = hipEventCreateWithFlags(&c->done, hipEventDisableTiming) == hipSuccess;
+        if (ok) {
+            // some room to grow, within what is kept
+            const size_t nb = bytes > kCutKeep ? bytes : (bytes + bytes / 4 < kCutKeep ? bytes + bytes / 4 : kCutKeep);
+            ok = device_alloc(&c->p, nb) == hipSuccess;
+            c->bytes = ok ? nb : 0;
+            if (!ok) c->p = nullptr;
+        }
     }
     if (!ok) {
         (void)hipGetLastError();

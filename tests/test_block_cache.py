@@ -147,6 +147,7 @@ def _free_bytes(bh):
 def test_trim_gives_back(bh):
     """What the library keeps goes back on request: freed blocks, and the block paths' buffers of every thread,
     one that lives on included; later calls work as before."""
+    import gc
     import threading
 
     n, kl, ku = 200000, 4, 4
@@ -160,6 +161,7 @@ def test_trim_gives_back(bh):
         return d.numpy()
 
     first = factor()
+    gc.collect()  # arrays that earlier tests left
     bh.trim()
     base = _free_bytes(bh)
     a = bh.DeviceArray((64 << 20,), np.uint8)

@@ -250,3 +250,23 @@ def test_laplacians_are_not_tried(bh, dtype, uplo, ldl, n, kd):
         else:
             bh._lib.call(f"bh_{FP[dtype]}pbtrf", uplo.encode(), n, kd, x.ptr, kd + 1, C.byref(info))
         assert info.value == 0 and verdict(bh)[0] == want, scale
+
+
+@pytest.mark.parametrize("uplo,trans", [("U", "N"), ("L", "T")])
+def test_impulse(bh, monkeypatch, uplo, trans):
+    """A right-hand side that is zero but for one entry: the tail of the solution is what a block among the zeros
+    cannot know.  The seams differ and the result is the sequential kernel's."""
+    n, k = 20000, 4
+    a = bh.DeviceArray.from_numpy(_tri(n, k, uplo == "U", np.float64, 1.5))
+    b = np.zeros(n)
+    b[n - 5000] = 1
+    out = []
+    for cut in (True, False):
+        if not cut:
+            monkeypatch.setenv("BANDEDHIP_CUT", "off")
+        x = bh.DeviceArray.from_numpy(b)
+        bh._lib.call("bh_dtbsv", uplo.encode(), trans.encode(), b"N", n, k, a.ptr, k + 1, x.ptr, 1)
+        assert verdict(bh)[0] == (DIFFERED if cut else NONE)
+        out.append(x.numpy())
+    assert out[0].tobytes() == out[1].tobytes()
+    assert np.count_nonzero(out[0]) > 20 * k + 64 * 2  # a tail longer than the lead-in
