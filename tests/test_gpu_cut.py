@@ -328,3 +328,39 @@ def test_stream_destroyed_and_another_created(bh, monkeypatch):
     assert hip.hipDeviceSynchronize() == 0
     for g, w in zip(got, want):
         _same((g.numpy(),), (w.numpy(),))
+
+
+def test_kept_buffer_used_while_another_stream_is_captured(bh, monkeypatch):
+    """The second and third call of a thread take its buffer again, while another stream is captured in the global
+    mode: that capture stays valid, and the results are those outside of it."""
+    monkeypatch.delenv("BANDEDHIP_CUT", raising=False)
+    hip = C.CDLL(bh._lib.LIB_PATH)
+    n, k = 30011, 3
+    ab = np.ones((k + 1, n), order="F")
+    ab[k] = 9
+    A, b = bh.DeviceArray.from_numpy(ab), np.random.default_rng(4).standard_normal(n)
+    xs = [bh.DeviceArray.from_numpy(b) for _ in range(4)]
+    errors = []
+
+    def solve(x):
+        try:
+            bh._lib.call("bh_dtbsv", b"U", b"N", b"N", n, k, A.ptr, k + 1, x.ptr, 1)
+        except Exception as e:
+            errors.append(e)
+
+    solve(xs[0])
+    bh.sync()
+    a, g = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(a)) == 0
+    assert hip.hipStreamBeginCapture(a, C.c_int(0)) == 0
+    t = threading.Thread(target=lambda: [solve(x) for x in xs[1:]])
+    t.start()
+    t.join()
+    assert hip.hipStreamEndCapture(a, C.byref(g)) == 0
+    if g.value:
+        assert hip.hipGraphDestroy(g) == 0
+    assert hip.hipStreamDestroy(a) == 0
+    assert not errors
+    want = xs[0].numpy()
+    for x in xs[1:]:
+        _same((x.numpy(),), (want,))
